@@ -171,6 +171,15 @@ int mdx_debug_attn_decode(int nq, int nkv, int hd, int pos, int rope_style, floa
  * rows [0, S+M) (the batch's own K/V already appended). */
 int mdx_debug_attn_prefill(int nq, int nkv, int hd, int S, int M, const float* q,
                            const uint16_t* k16, const uint16_t* v16, float* out);
+/* The same three through the kernels of a prompt longer than 64 rows (any M;
+ * K a multiple of 32). */
+int mdx_debug_long_gemm(int kind, int M, int K, int N, const void* w, const float* scales,
+                        const float* x, float* y);
+int mdx_debug_long_residual(int kind, int M, int K, int N, const void* w, const float* scales,
+                            const float* x, float* hidden, const float* norm_w, float eps,
+                            uint16_t* x16_out);
+int mdx_debug_long_attn(int nq, int nkv, int hd, int S, int M, const float* q,
+                        const uint16_t* k16, const uint16_t* v16, float* out);
 /* QK-norm + RoPE + KV append of one token at position pos through the
  * batch-prefill kernel: qkv fp32 [nq*hd + 2*nkv*hd]; returns q fp32 and
  * the fp16 k,v rows. */

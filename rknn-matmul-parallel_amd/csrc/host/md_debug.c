@@ -168,9 +168,9 @@ int mdx_time_gemv(int kind, int K, int N, int copies, int iters, float* avg_us) 
     return rc ? MATMUL_DECODER_ERR_RKNN : 0;
 }
 
-int mdx_debug_gemm(int kind, int M, int K, int N, const void* w, const float* scales,
-                   const float* x, float* y) {
-    if (kind < 0 || kind > 2 || M <= 0 || M > 64 || K <= 0 || N <= 0 || !w || !x || !y)
+static int debug_gemm(int lng, int kind, int M, int K, int N, const void* w, const float* scales,
+                      const float* x, float* y) {
+    if (kind < 0 || kind > 2 || M <= 0 || (!lng && M > 64) || K <= 0 || N <= 0 || !w || !x || !y)
         return MATMUL_DECODER_ERR_INVALID_ARG;
     dbg_scope s;
     int rc = scope_open(&s);
@@ -185,16 +185,27 @@ int mdx_debug_gemm(int kind, int M, int K, int N, const void* w, const float* sc
     if (!rc) rc = mdxrt_fill_u32(scr, 0u, mdx_gemm_scratch_floats(M, N, K), s.stream);
     if (!rc) rc = mdxrt_h2d(dx, x, (size_t)M * K * 4);
     if (!rc) rc = mdx_launch_to_f16(dx, M * K, dx16, s.stream);
-    if (!rc) rc = mdx_launch_gemm(dx16, M, &d, 0, dy, scr, s.stream);
+    if (!rc) rc = lng ? mdx_launch_long_gemm(dx16, M, &d, 0, dy, s.stream)
+                      : mdx_launch_gemm(dx16, M, &d, 0, dy, scr, s.stream);
     if (!rc) rc = mdxrt_stream_sync(s.stream);
     if (!rc) rc = mdxrt_d2h(y, dy, (size_t)M * N * 4);
     return scope_close(&s, rc);
 }
 
-int mdx_debug_gemm_residual(int kind, int M, int K, int N, const void* w, const float* scales,
-                            const float* x, float* hidden, const float* norm_w, float eps,
-                            uint16_t* x16_out) {
-    if (kind < 0 || kind > 2 || M <= 0 || M > 64 || K <= 0 || N <= 0 || !w || !x || !hidden ||
+int mdx_debug_gemm(int kind, int M, int K, int N, const void* w, const float* scales,
+                   const float* x, float* y) {
+    return debug_gemm(0, kind, M, K, N, w, scales, x, y);
+}
+
+int mdx_debug_long_gemm(int kind, int M, int K, int N, const void* w, const float* scales,
+                        const float* x, float* y) {
+    return debug_gemm(1, kind, M, K, N, w, scales, x, y);
+}
+
+static int debug_residual(int lng, int kind, int M, int K, int N, const void* w, const float* scales,
+                          const float* x, float* hidden, const float* norm_w, float eps,
+                          uint16_t* x16_out) {
+    if (kind < 0 || kind > 2 || M <= 0 || (!lng && M > 64) || K <= 0 || N <= 0 || !w || !x || !hidden ||
         (norm_w && !x16_out))
         return MATMUL_DECODER_ERR_INVALID_ARG;
     dbg_scope s;
@@ -207,17 +218,31 @@ int mdx_debug_gemm_residual(int kind, int M, int K, int N, const void* w, const 
     float* dh = rc ? NULL : (float*)dalloc(&s, (size_t)M * N * 4);
     float* dnw = (rc || !norm_w) ? NULL : (float*)dalloc(&s, (size_t)N * 4);
     uint16_t* dout = (rc || !norm_w) ? NULL : (uint16_t*)dalloc(&s, (size_t)M * N * 2);
-    float* scr = rc ? NULL : (float*)dalloc(&s, mdx_gemm_scratch_floats(M, N, K) * 4);
+    const size_t scr_n = lng ? mdx_long_scratch_floats(M, N) : mdx_gemm_scratch_floats(M, N, K);
+    float* scr = rc ? NULL : (float*)dalloc(&s, scr_n * 4);
     if (!rc && (!dx || !dx16 || !dh || !scr || (norm_w && (!dnw || !dout)))) rc = MATMUL_DECODER_ERR_MEMORY;
     if (!rc) rc = mdxrt_h2d(dx, x, (size_t)M * K * 4);
     if (!rc) rc = mdxrt_h2d(dh, hidden, (size_t)M * N * 4);
     if (!rc && norm_w) rc = mdxrt_h2d(dnw, norm_w, (size_t)N * 4);
     if (!rc) rc = mdx_launch_to_f16(dx, M * K, dx16, s.stream);
-    if (!rc) rc = mdx_launch_gemm_residual_norm(dx16, M, &d, dh, dnw, eps, dout, scr, s.stream);
+    if (!rc) rc = lng ? mdx_launch_long_residual_norm(dx16, M, &d, dh, dnw, eps, dout, scr, s.stream)
+                      : mdx_launch_gemm_residual_norm(dx16, M, &d, dh, dnw, eps, dout, scr, s.stream);
     if (!rc) rc = mdxrt_stream_sync(s.stream);
     if (!rc) rc = mdxrt_d2h(hidden, dh, (size_t)M * N * 4);
     if (!rc && norm_w) rc = mdxrt_d2h(x16_out, dout, (size_t)M * N * 2);
     return scope_close(&s, rc);
+}
+
+int mdx_debug_gemm_residual(int kind, int M, int K, int N, const void* w, const float* scales,
+                            const float* x, float* hidden, const float* norm_w, float eps,
+                            uint16_t* x16_out) {
+    return debug_residual(0, kind, M, K, N, w, scales, x, hidden, norm_w, eps, x16_out);
+}
+
+int mdx_debug_long_residual(int kind, int M, int K, int N, const void* w, const float* scales,
+                            const float* x, float* hidden, const float* norm_w, float eps,
+                            uint16_t* x16_out) {
+    return debug_residual(1, kind, M, K, N, w, scales, x, hidden, norm_w, eps, x16_out);
 }
 
 static int upload_state(dbg_scope* s, int pos, mdx_state** d_state) {
@@ -301,8 +326,8 @@ int mdx_debug_attn_decode(int nq, int nkv, int hd, int pos, int rope_style, floa
     return scope_close(&s, rc);
 }
 
-int mdx_debug_attn_prefill(int nq, int nkv, int hd, int S, int M, const float* q,
-                           const uint16_t* k16, const uint16_t* v16, float* out) {
+static int debug_attn(int lng, int nq, int nkv, int hd, int S, int M, const float* q,
+                      const uint16_t* k16, const uint16_t* v16, float* out) {
     if (nq <= 0 || nkv <= 0 || hd <= 0 || S < 0 || M <= 0 || !q || !k16 || !v16 || !out)
         return MATMUL_DECODER_ERR_INVALID_ARG;
     dbg_scope s;
@@ -319,13 +344,24 @@ int mdx_debug_attn_prefill(int nq, int nkv, int hd, int S, int M, const float* q
     if (!rc) rc = mdxrt_h2d(dq, q, (size_t)M * qd * 4);
     if (!rc) rc = mdxrt_h2d(dk, k16, (size_t)L * kvd * 2);
     if (!rc) rc = mdxrt_h2d(dv, v16, (size_t)L * kvd * 2);
-    if (!rc) rc = mdx_launch_attn_prefill(st, dq, M, dk, dv, nq, nkv, hd, o16, s.stream);
+    if (!rc) rc = lng ? mdx_launch_long_attn(S, dq, M, dk, dv, nq, nkv, hd, o16, s.stream)
+                      : mdx_launch_attn_prefill(st, dq, M, dk, dv, nq, nkv, hd, o16, s.stream);
     if (!rc) rc = mdxrt_stream_sync(s.stream);
     uint16_t* h = (uint16_t*)malloc((size_t)M * qd * 2);
     if (!rc) rc = h ? mdxrt_d2h(h, o16, (size_t)M * qd * 2) : MATMUL_DECODER_ERR_MEMORY;
     if (!rc) widen(h, out, (size_t)M * qd);
     free(h);
     return scope_close(&s, rc);
+}
+
+int mdx_debug_attn_prefill(int nq, int nkv, int hd, int S, int M, const float* q,
+                           const uint16_t* k16, const uint16_t* v16, float* out) {
+    return debug_attn(0, nq, nkv, hd, S, M, q, k16, v16, out);
+}
+
+int mdx_debug_long_attn(int nq, int nkv, int hd, int S, int M, const float* q,
+                        const uint16_t* k16, const uint16_t* v16, float* out) {
+    return debug_attn(1, nq, nkv, hd, S, M, q, k16, v16, out);
 }
 
 int mdx_debug_qk_rope(int nq, int nkv, int hd, int pos, int rope_style, float theta, float eps,

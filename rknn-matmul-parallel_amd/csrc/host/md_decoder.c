@@ -39,6 +39,8 @@ struct MatmulDecoderContext {
     int max_seq, seq_len;
     int d, nq, nkv, hd, qd, kvd, F, V, L;
     int n_lm, lm_vocab, max_m, max_splits;
+    int long_m;              /* rows per pass of a prompt longer than max_m (0: none) */
+    int last_row;            /* d_bhidden row of the last prefilled position */
     void* stream;
     uint8_t* arena;
     size_t arena_size, arena_used;
@@ -377,20 +379,22 @@ static int layout(MatmulDecoderContext* c, const md_source* s) {
     CARVE(c->d_act16, (size_t)c->F * 2);
     CARVE(c->d_partial, mdx_lmhead_scratch_bytes());
     CARVE(c->d_xbuf, mdx_persist_xbuf_bytes());
-    const int mm = c->max_m;
+    const int mm = c->long_m > c->max_m ? c->long_m : c->max_m;
+    const int mq = c->hd > 128 ? mm : c->max_m;   /* head_dim 256: qkv and RoPE are two launches */
     const int kmax = c->F > c->qd ? (c->F > c->d ? c->F : c->d) : (c->qd > c->d ? c->qd : c->d);
     CARVE(c->d_bhidden, (size_t)mm * c->d * 4);
-    CARVE(c->d_bqkv, (size_t)mm * (c->qd + 2 * c->kvd) * 4);
+    CARVE(c->d_bqkv, (size_t)mq * (c->qd + 2 * c->kvd) * 4);
     CARVE(c->d_bq, (size_t)mm * c->qd * 4);
     CARVE(c->d_bx16, (size_t)mm * kmax * 2);
     CARVE(c->d_battn16, (size_t)mm * c->qd * 2);
     CARVE(c->d_bact16, (size_t)mm * c->F * 2);
     {
-        size_t g = mdx_gemm_scratch_floats(mm, c->qd + 2 * c->kvd, c->d);
+        size_t g = mdx_gemm_scratch_floats(c->max_m, c->qd + 2 * c->kvd, c->d);
         size_t t;
-        t = mdx_gemm_scratch_floats(mm, c->d, c->qd); if (t > g) g = t;
-        t = mdx_gemm_scratch_floats(mm, 2 * c->F, c->d); if (t > g) g = t;
-        t = mdx_gemm_scratch_floats(mm, c->d, c->F); if (t > g) g = t;
+        t = mdx_gemm_scratch_floats(c->max_m, c->d, c->qd); if (t > g) g = t;
+        t = mdx_gemm_scratch_floats(c->max_m, 2 * c->F, c->d); if (t > g) g = t;
+        t = mdx_gemm_scratch_floats(c->max_m, c->d, c->F); if (t > g) g = t;
+        if (c->long_m) { t = mdx_long_scratch_floats(c->long_m, c->d); if (t > g) g = t; }
         CARVE(c->d_gscr, g * 4);
     }
 #undef CARVE
@@ -567,6 +571,39 @@ static int run_prefill(MatmulDecoderContext* c, int M, void* s) {
         if (!rc)
             rc = mdx_launch_gemm_residual_norm(c->d_bact16, M, &ly->down, c->d_bhidden, next_norm,
                                                eps, c->d_bx16, c->d_gscr, s);
+    }
+    if (!rc) rc = mdx_launch_advance(c->d_state, M, s);
+    return rc;
+}
+
+/* The same for any number of rows at positions pos0.. (the tiled kernels of
+ * mdx_prefill_long.hip). */
+static int run_prefill_long(MatmulDecoderContext* c, int M, int pos0, void* s) {
+    const float eps = c->config.rms_eps;
+    int rc = mdx_launch_rmsnorm_rows(c->d_bhidden, c->layers[0].in_norm, eps, M, c->d, c->d_bx16, s);
+    for (int l = 0; l < c->L && rc == 0; l++) {
+        md_layer* ly = &c->layers[l];
+        const float* next_norm = l + 1 < c->L ? c->layers[l + 1].in_norm : NULL;
+        if (c->hd <= 128) {
+            rc = mdx_launch_long_qkv_rope(c->d_bx16, M, &ly->qkv, pos0, ly->q_norm, ly->k_norm, eps, c->d_cos,
+                                          c->d_sin, c->nq, c->nkv, c->hd, c->config.rope_style, c->d_bq,
+                                          ly->kc, ly->vc, s);
+        } else {
+            rc = mdx_launch_long_gemm(c->d_bx16, M, &ly->qkv, 0, c->d_bqkv, s);
+            if (!rc)
+                rc = mdx_launch_qk_rope_append_rows(c->d_state, c->d_bqkv, M, ly->q_norm, ly->k_norm, eps,
+                                                    c->d_cos, c->d_sin, c->nq, c->nkv, c->hd,
+                                                    c->config.rope_style, c->d_bq, ly->kc, ly->vc, s);
+        }
+        if (!rc)
+            rc = mdx_launch_long_attn(pos0, c->d_bq, M, ly->kc, ly->vc, c->nq, c->nkv, c->hd, c->d_battn16, s);
+        if (!rc)
+            rc = mdx_launch_long_residual_norm(c->d_battn16, M, &ly->o, c->d_bhidden, ly->post_norm, eps,
+                                               c->d_bx16, c->d_gscr, s);
+        if (!rc) rc = mdx_launch_long_gemm(c->d_bx16, M, &ly->gu, 1, c->d_bact16, s);
+        if (!rc)
+            rc = mdx_launch_long_residual_norm(c->d_bact16, M, &ly->down, c->d_bhidden, next_norm, eps,
+                                               c->d_bx16, c->d_gscr, s);
     }
     if (!rc) rc = mdx_launch_advance(c->d_state, M, s);
     return rc;
@@ -850,6 +887,9 @@ static MatmulDecoderContext* create_common(const MatmulDecoderConfig* config,
                           : c->V;
     int mm = config->max_batch_prefill > 0 ? config->max_batch_prefill : 64;
     c->max_m = mm > 64 ? 64 : mm;
+    /* a chunk size below 64 is kept to; otherwise a longer prompt goes in
+     * passes of up to 2048 rows (about 80 MB of activations at d = 1024) */
+    c->long_m = c->max_m == 64 && max_seq_len > 64 ? (max_seq_len < 2048 ? max_seq_len : 2048) : 0;
     c->max_splits = mdx_attn_max_splits(max_seq_len);
     {
         const char* e = getenv("MDX_GRAPHS");
@@ -1314,19 +1354,25 @@ int matmul_decoder_step_head(MatmulDecoderContext* c, int token_id, const float*
 }
 
 static int prefill_chunk(MatmulDecoderContext* c, const float* emb, int M) {
-    memcpy(c->h_io, emb, (size_t)M * c->d * 4);
     memset(c->h_state, 0, sizeof(mdx_state));
     c->h_state->pos = c->seq_len;
-    int rc = mdxrt_h2d_async(c->d_bhidden, c->h_io, (size_t)M * c->d * 4, c->stream);
-    if (!rc) rc = mdxrt_h2d_async(c->d_state, c->h_state, sizeof(mdx_state), c->stream);
-    void* g = rc ? NULL : prefill_graph(c, M);
-    if (!rc) rc = g ? mdxrt_graph_launch(g, c->stream) : run_prefill(c, M, c->stream);
+    int rc = mdxrt_h2d_async(c->d_state, c->h_state, sizeof(mdx_state), c->stream);
+    if (M <= c->max_m) {
+        memcpy(c->h_io, emb, (size_t)M * c->d * 4);
+        if (!rc) rc = mdxrt_h2d_async(c->d_bhidden, c->h_io, (size_t)M * c->d * 4, c->stream);
+        void* g = rc ? NULL : prefill_graph(c, M);
+        if (!rc) rc = g ? mdxrt_graph_launch(g, c->stream) : run_prefill(c, M, c->stream);
+    } else {
+        if (!rc) rc = mdxrt_h2d_async(c->d_bhidden, emb, (size_t)M * c->d * 4, c->stream);
+        if (!rc) rc = run_prefill_long(c, M, c->seq_len, c->stream);
+    }
     if (!rc) rc = mdxrt_stream_sync(c->stream);
     if (rc) {
         fprintf(stderr, "[BatchPrefill] failed: %s\n", mdxrt_last_error());
         return MATMUL_DECODER_ERR_RKNN;
     }
     c->seq_len += M;
+    c->last_row = M - 1;
     return 0;
 }
 
@@ -1337,8 +1383,14 @@ int matmul_decoder_prefill_batch(MatmulDecoderContext* c, const float* embedding
                 M, c->max_seq);
         return MATMUL_DECODER_ERR_INVALID_ARG;
     }
-    for (int off = 0; off < M; off += c->max_m) {
-        const int n = M - off < c->max_m ? M - off : c->max_m;
+    /* equal passes (one of a few rows would read all weights for them) */
+    int step = c->max_m;
+    if (M > c->max_m && c->long_m) {
+        const int n = (M + c->long_m - 1) / c->long_m;
+        step = (M + n - 1) / n;
+    }
+    for (int off = 0; off < M; off += step) {
+        const int n = M - off < step ? M - off : step;
         int rc = prefill_chunk(c, embeddings + (size_t)off * c->d, n);
         if (rc) return rc;
     }
@@ -1495,8 +1547,7 @@ int mdx_prefill_logits(MatmulDecoderContext* c, const float* embeddings, int M, 
     if (!c || c->n_lm > 1) return MATMUL_DECODER_ERR_INVALID_ARG;
     int rc = matmul_decoder_prefill_batch(c, embeddings, M);
     if (rc) return rc;
-    const int last = (M - 1) % c->max_m;
-    rc = mdx_launch_copy_row(c->d_bhidden, last, c->d, c->d_hidden, c->stream);
+    rc = mdx_launch_copy_row(c->d_bhidden, c->last_row, c->d, c->d_hidden, c->stream);
     if (!rc) rc = run_head(c, &c->lm, NULL, 0, c->stream);
     if (!rc && logits) rc = mdxrt_d2h_async(c->h_io, c->d_logits, (size_t)c->V * 4, c->stream);
     if (!rc) rc = mdxrt_d2h_async(c->h_state, c->d_state, sizeof(mdx_state), c->stream);

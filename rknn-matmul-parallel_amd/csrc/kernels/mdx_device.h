@@ -266,6 +266,35 @@ int mdx_launch_attn_prefill(const mdx_state* state, const float* q, int M,
                             const uint16_t* k_cache, const uint16_t* v_cache, int nq, int nkv,
                             int hd, uint16_t* out16, void* stream);
 
+/* The finish of a split residual projection: hidden[m][n] += (sum of the ns
+ * partials, part[s][rows][N], in split order) x scale, then the row's
+ * RMSNorm as above. */
+int mdx_launch_residual_norm(const float* part, int ns, int rows, int M, int N, const float* scale,
+                             float* hidden, const float* norm_w, float eps, uint16_t* x16_out, void* stream);
+
+/* ---- batch prefill, any M (mdx_prefill_long.hip) ---- */
+
+/* 1 when the long-prefill projections serve w (K a multiple of 32). */
+int mdx_long_ok(const mdx_wdesc* w);
+/* Y = X16[M][K] . W^T (x scale): fp32 y[M][N], or with swiglu the fp16
+ * act[M][N/2] of rows [0,N/2) gate and [N/2,N) up. */
+int mdx_launch_long_gemm(const uint16_t* x16, int M, const mdx_wdesc* w, int swiglu, void* out, void* stream);
+/* Residual projection + next RMSNorm, as mdx_launch_gemm_residual_norm;
+ * scratch: mdx_long_scratch_floats(M, N) floats. */
+size_t mdx_long_scratch_floats(int M, int N);
+int mdx_launch_long_residual_norm(const uint16_t* x16, int M, const mdx_wdesc* w, float* hidden,
+                                  const float* norm_w, float eps, uint16_t* x16_out, float* scratch,
+                                  void* stream);
+/* qkv projection, QK-norm, RoPE and append in one kernel (hd 64 or 128): rows
+ * t < M at positions pos0 + t. */
+int mdx_launch_long_qkv_rope(const uint16_t* x16, int M, const mdx_wdesc* w, int pos0, const float* q_norm,
+                             const float* k_norm, float eps, const float* cos_t, const float* sin_t, int nq,
+                             int nkv, int hd, int rope_style, float* q_out, uint16_t* k_cache,
+                             uint16_t* v_cache, void* stream);
+/* Causal attention as mdx_launch_attn_prefill, at positions pos0 + t. */
+int mdx_launch_long_attn(int pos0, const float* q, int M, const uint16_t* k_cache, const uint16_t* v_cache,
+                         int nq, int nkv, int hd, uint16_t* out16, void* stream);
+
 /* Copy row M-1 of x[M][d] to dst[d] (last-token hidden after prefill). */
 int mdx_launch_copy_row(const float* x, int row, int d, float* dst, void* stream);
 

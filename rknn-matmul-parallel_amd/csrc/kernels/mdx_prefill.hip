@@ -497,7 +497,7 @@ __global__ __launch_bounds__(NW * 64) void k_gemm_s(const uint16_t* __restrict__
 // Split-K finish for the o and down projections: y = sum of the split
 // partials (split order) x scale; hidden += y (the residual); then the next
 // RMSNorm of the row, x16 = fp16((hidden * rms) * norm_w) (skipped when norm_w
-// is NULL).  grid = M rows, 256 threads.
+// is NULL).  A split's partials are rows x N.  grid = M rows, 256 threads.
 constexpr int kMaxSplits = 16;
 
 // R > 0: N == 1024 * R, thread t owns columns 4t..4t+3 (+1024 per round), and
@@ -505,7 +505,7 @@ constexpr int kMaxSplits = 16;
 // weights are requested with the partials, so the block waits for memory once.
 // R == 0: any N (a multiple of 4), rounds looped at run time.
 template <int R>
-__global__ __launch_bounds__(256) void k_residual_norm(const float* part, int ns, int N,
+__global__ __launch_bounds__(256) void k_residual_norm(const float* part, int ns, int rows, int N,
                                                        const float* scale, float* hidden,
                                                        const float* norm_w, float eps,
                                                        uint16_t* x16) {
@@ -523,7 +523,7 @@ __global__ __launch_bounds__(256) void k_residual_norm(const float* part, int ns
         float4 p[kMaxSplits];
 #pragma unroll
         for (int sp = 0; sp < kMaxSplits; sp++)
-            if (sp < ns) p[sp] = *reinterpret_cast<const float4*>(part + ((size_t)sp * kMaxM + m) * N + c);
+            if (sp < ns) p[sp] = *reinterpret_cast<const float4*>(part + ((size_t)sp * rows + m) * N + c);
         const float4 h0 = *reinterpret_cast<const float4*>(hr + c);
         const float4 sc = scale ? *reinterpret_cast<const float4*>(scale + c) : make_float4(1.f, 1.f, 1.f, 1.f);
         float4 y = p[0];
@@ -1022,10 +1022,16 @@ int mdx_launch_gemm_residual_norm(const uint16_t* x16, int M, const mdx_wdesc* w
         rc = gemm_launch(x16, M, w, 0, nullptr, scratch, ns, stream);
     }
     if (rc) return rc;
-    const int R = w->N % 1024 == 0 ? w->N / 1024 : 0;
+    return mdx_launch_residual_norm(scratch, ns, kMaxM, M, w->N, w->scale, hidden, norm_w, eps, x16_out, stream);
+}
+
+int mdx_launch_residual_norm(const float* part, int ns, int rows, int M, int N, const float* scale,
+                             float* hidden, const float* norm_w, float eps, uint16_t* x16_out, void* stream) {
+    if (N % 4 || ns < 1 || ns > kMaxSplits || M <= 0) return -1;
+    const int R = N % 1024 == 0 ? N / 1024 : 0;
     auto kern = R == 1 ? k_residual_norm<1> : R == 2 ? k_residual_norm<2> : R == 4 ? k_residual_norm<4>
                                                                                   : k_residual_norm<0>;
-    hipLaunchKernelGGL(kern, dim3(M), dim3(256), 0, (hipStream_t)stream, scratch, ns, w->N, w->scale,
+    hipLaunchKernelGGL(kern, dim3(M), dim3(256), 0, (hipStream_t)stream, part, ns, rows, N, scale,
                        hidden, norm_w, eps, x16_out);
     return hipGetLastError() == hipSuccess ? 0 : -4;
 }

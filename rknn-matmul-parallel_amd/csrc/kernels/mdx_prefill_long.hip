@@ -1,0 +1,767 @@
+// mdx_prefill_long.hip — batch prefill of more than 64 rows, gfx950.
+//
+// The kernels of mdx_prefill.hip take 64 rows per pass over the weights and
+// give every query row an attention block of its own.  A longer prompt has
+// enough rows to tile both operands: here the projections are LDS-tiled MFMA
+// GEMMs over all rows (each weight read once per row tile, int8/int4 widened
+// to fp16 once per block as they are staged), and attention runs 64 query
+// rows of one KV head against each staged K/V tile on MFMA.  A prompt of 2000
+// rows through 28 fp16 layers (hidden 1024) and 32 tokens: 91.0 -> 23.3 ms;
+// 4000 rows through 2 int4 layers and 32 tokens: 20.1 -> 4.1 ms; 203 rows
+// through 4 int8 layers and 16 tokens: 2.23 -> 1.77 ms.
+#include <hip/hip_runtime.h>
+
+#include <cmath>
+
+#include "mdx_common.h"
+#include "mdx_device.h"
+#include "mdx_gemm_tile.h"
+
+using namespace mdx;
+
+namespace {
+
+constexpr int kKT = 64;            // k per LDS stage
+constexpr int kStageChunks = kKT / 8;   // 16-byte chunks per LDS row
+
+// Where the tile's 16-byte chunk of row r goes: chunks are permuted within the
+// row by the row index, so the 16 rows of an MFMA fragment read spread over
+// the banks without padding.
+__device__ __forceinline__ int lds_chunk(int row, int chunk) {
+    return row * kStageChunks + (chunk ^ (row & 7));
+}
+
+// Block id -> work item: ids id, id + 8, ... run on one XCD (one L2); each XCD
+// takes a contiguous run of items.  A bijection for any count.
+__device__ __forceinline__ int xcd_item(int id, int n) {
+    const int q = n >> 3, r = n & 7, x = id & 7, i = id >> 3;
+    return x * q + min(x, r) + i;
+}
+
+enum LongEpi { LE_STORE = 0, LE_PART = 1, LE_SWIGLU = 2, LE_ROPE = 3 };
+
+struct LongArgs {
+    const uint16_t* x16;      // [M][K]
+    const uint8_t* w;         // W^T rows
+    const float* scale;       // [N] or NULL
+    int M, K, N;
+    int tiles_m, tiles_n, splits, per_split;   // per_split: LDS stages per split
+    float* out;               // LE_STORE [M][N]; LE_PART [splits][M][N], unscaled
+    uint16_t* out16;          // LE_SWIGLU [M][N/2]
+    // LE_ROPE
+    int pos0, nq, nkv, style;
+    const float* q_norm;
+    const float* k_norm;
+    float eps;
+    const float* cos_t;
+    const float* sin_t;
+    float* q_out;             // [M][nq*hd]
+    uint16_t* kc;             // [max_seq][nkv*hd]
+    uint16_t* vc;
+};
+
+// Weight row of tile row c (0..BN-1): consecutive rows, or for SwiGLU
+// alternating runs of 16 gate rows and the 16 up rows of the same features.
+template <int BN>
+__device__ __forceinline__ int long_row(int tile, int c, bool swiglu, int N) {
+    if (!swiglu) return tile * BN + c;
+    const int f = tile * (BN / 2) + (c >> 5) * 16 + (c & 15);
+    return f < N / 2 ? ((c & 16) ? N / 2 + f : f) : N;
+}
+
+// QK-norm + RoPE + append of the head slices a wave holds.  acc[t][j]: weight
+// columns 16t + 4g + i (t within the wave's NT tiles) of row m; a head is HD
+// consecutive columns, all in this lane and its three g-partners.
+template <int HD, int NT>
+__device__ __forceinline__ void rope_store(const LongArgs& a, float4_t (&v)[NT], int col0, int m, int g,
+                                           bool store) {
+    constexpr int TH = HD / 16;               // tiles per head
+    const int qd = a.nq * HD, kvd = a.nkv * HD;
+    const size_t pos = (size_t)a.pos0 + m;
+#pragma unroll
+    for (int h = 0; h < NT / TH; h++) {
+        const int c0 = col0 + h * HD;         // the head's first column
+        if (c0 >= a.N) break;
+        float4_t* x = v + h * TH;
+        if (c0 >= qd + kvd) {
+            uint16_t* dst = a.vc + pos * kvd + (c0 - qd - kvd);
+#pragma unroll
+            for (int t = 0; t < TH; t++) {
+                uint2 o;
+                o.x = (uint32_t)f32_to_f16_bits(x[t][0]) | ((uint32_t)f32_to_f16_bits(x[t][1]) << 16);
+                o.y = (uint32_t)f32_to_f16_bits(x[t][2]) | ((uint32_t)f32_to_f16_bits(x[t][3]) << 16);
+                if (store) *reinterpret_cast<uint2*>(dst + 16 * t + 4 * g) = o;
+            }
+            continue;
+        }
+        const bool is_q = c0 < qd;
+        const float* nw = is_q ? a.q_norm : a.k_norm;
+        if (nw) {
+            float ss = 0.0f;
+#pragma unroll
+            for (int t = 0; t < TH; t++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) ss += x[t][i] * x[t][i];
+            ss = rows_sum4(ss);
+            const float rms = 1.0f / sqrtf(ss / (float)HD + a.eps);
+#pragma unroll
+            for (int t = 0; t < TH; t++) {
+                const float4 w = *reinterpret_cast<const float4*>(nw + 16 * t + 4 * g);
+                x[t][0] = (x[t][0] * rms) * w.x;
+                x[t][1] = (x[t][1] * rms) * w.y;
+                x[t][2] = (x[t][2] * rms) * w.z;
+                x[t][3] = (x[t][3] * rms) * w.w;
+            }
+        }
+        const float* cr = a.cos_t + pos * (HD / 2);
+        const float* sr = a.sin_t + pos * (HD / 2);
+        if (a.style == 0) {
+            // pairs (2i, 2i+1)
+#pragma unroll
+            for (int t = 0; t < TH; t++) {
+                const float2 c = *reinterpret_cast<const float2*>(cr + 8 * t + 2 * g);
+                const float2 s = *reinterpret_cast<const float2*>(sr + 8 * t + 2 * g);
+                const float a0 = x[t][0], b0 = x[t][1], a1 = x[t][2], b1 = x[t][3];
+                x[t][0] = a0 * c.x - b0 * s.x;
+                x[t][1] = b0 * c.x + a0 * s.x;
+                x[t][2] = a1 * c.y - b1 * s.y;
+                x[t][3] = b1 * c.y + a1 * s.y;
+            }
+        } else {
+            // pairs (i, i + HD/2)
+#pragma unroll
+            for (int t = 0; t < TH / 2; t++) {
+                const float4 c = *reinterpret_cast<const float4*>(cr + 16 * t + 4 * g);
+                const float4 s = *reinterpret_cast<const float4*>(sr + 16 * t + 4 * g);
+                const float cc[4] = {c.x, c.y, c.z, c.w}, sc[4] = {s.x, s.y, s.z, s.w};
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const float x0 = x[t][i], x1 = x[t + TH / 2][i];
+                    x[t][i] = x0 * cc[i] - x1 * sc[i];
+                    x[t + TH / 2][i] = x1 * cc[i] + x0 * sc[i];
+                }
+            }
+        }
+        if (!store) continue;
+        if (is_q) {
+            float* dst = a.q_out + (size_t)m * qd + c0;
+#pragma unroll
+            for (int t = 0; t < TH; t++)
+                *reinterpret_cast<float4*>(dst + 16 * t + 4 * g) = make_float4(x[t][0], x[t][1], x[t][2], x[t][3]);
+        } else {
+            uint16_t* dst = a.kc + pos * kvd + (c0 - qd);
+#pragma unroll
+            for (int t = 0; t < TH; t++) {
+                uint2 o;
+                o.x = (uint32_t)f32_to_f16_bits(x[t][0]) | ((uint32_t)f32_to_f16_bits(x[t][1]) << 16);
+                o.y = (uint32_t)f32_to_f16_bits(x[t][2]) | ((uint32_t)f32_to_f16_bits(x[t][3]) << 16);
+                *reinterpret_cast<uint2*>(dst + 16 * t + 4 * g) = o;
+            }
+        }
+    }
+}
+
+// ---- projections: LDS-tiled MFMA GEMM -----------------------------------------
+//
+// Block = 4 waves, one BN (weight rows) x BM (activation rows) tile; a stage
+// is 64 k of both panels in LDS (fp16, two buffers), staged through registers
+// PD stages ahead.  The weights are the MFMA A operand, the activations the B
+// operand, so a lane ends with 4 consecutive output columns of one row:
+// 16-byte stores, SwiGLU pairs and RoPE pairs in one lane.  Waves split the
+// tile WN x (4/WN).  Lane group g takes k 16g + 8s .. +7 of a stage at step s
+// for both operands.
+template <int KIND, int BM, int BN, int WN, int PD, int EPI, int HD>
+__global__ __launch_bounds__(256, 2) void k_long_gemm(LongArgs a) {
+    constexpr int WM = 4 / WN;
+    constexpr int NT = BN / WN / 16, MT = BM / WM / 16;   // 16x16 tiles per wave
+    constexpr int XU = BM * kStageChunks / 256;           // 16-byte loads per thread, activations
+    constexpr int KPU = KIND == MDX_W_F16 ? 8 : (KIND == MDX_W_I8 ? 16 : 32);   // k per weight load
+    constexpr int UPR = kKT / KPU;                        // weight loads per row
+    constexpr int WUN = BN * UPR, WU = (WUN + 255) / 256;
+    constexpr bool SWIGLU = EPI == LE_SWIGLU;
+    __shared__ uint4 xs[2][BM * kStageChunks];
+    __shared__ uint4 ws[2][BN * kStageChunks];
+
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int g = lane >> 4, c16 = lane & 15;
+    const int wn = wave % WN, wm = wave / WN;
+    const int item = xcd_item(blockIdx.x, gridDim.x);
+    const int tm = item % a.tiles_m, rest = item / a.tiles_m;
+    const int tn = rest % a.tiles_n, split = rest / a.tiles_n;
+    const int nst_all = (a.K + kKT - 1) / kKT;
+    const int s0 = split * a.per_split, s1 = min(nst_all, s0 + a.per_split);
+    const size_t row_bytes = KIND == MDX_W_F16 ? (size_t)a.K * 2 : (KIND == MDX_W_I8 ? (size_t)a.K : (size_t)a.K / 2);
+
+    // this thread's loads: rows past the edge repeat the last row (their
+    // results are not stored)
+    const uint16_t* xp[XU];
+    int xk[XU], xl[XU];
+#pragma unroll
+    for (int i = 0; i < XU; i++) {
+        const int u = tid + 256 * i, row = u / kStageChunks, ch = u % kStageChunks;
+        xk[i] = 8 * ch;
+        xl[i] = lds_chunk(row, ch);
+        xp[i] = a.x16 + (size_t)min(tm * BM + row, a.M - 1) * a.K + 8 * ch;
+    }
+    const uint8_t* wp[WU];
+    int wk[WU], wr[WU];
+#pragma unroll
+    for (int i = 0; i < WU; i++) {
+        const int u = min(tid + 256 * i, WUN - 1), row = u / UPR, ch = u % UPR;
+        wk[i] = KPU * ch;
+        wr[i] = row;
+        wp[i] = a.w + (size_t)min(long_row<BN>(tn, row, SWIGLU, a.N), a.N - 1) * row_bytes + (size_t)ch * 16;
+    }
+    uint4 xv[PD][XU], wv[PD][WU];
+    // K is a multiple of 32, so no load straddles it; those past it are zeros
+    auto load = [&](int d, int st) {
+        const int k0 = st * kKT;
+#pragma unroll
+        for (int i = 0; i < XU; i++)
+            xv[d][i] = k0 + xk[i] < a.K ? *reinterpret_cast<const uint4*>(xp[i] + k0) : make_uint4(0u, 0u, 0u, 0u);
+#pragma unroll
+        for (int i = 0; i < WU; i++)
+            wv[d][i] = k0 + wk[i] < a.K ? *reinterpret_cast<const uint4*>(wp[i] + (size_t)st * (16 * UPR))
+                                        : make_uint4(0u, 0u, 0u, 0u);
+    };
+    auto stash = [&](int d, int buf) {
+#pragma unroll
+        for (int i = 0; i < XU; i++) xs[buf][xl[i]] = xv[d][i];
+#pragma unroll
+        for (int i = 0; i < WU; i++) {
+            if (WUN % 256 != 0 && tid + 256 * i >= WUN) break;
+            half8_t b[KPU / 8];
+            widen_b<KIND>(wv[d][i], b);
+#pragma unroll
+            for (int s = 0; s < KPU / 8; s++)
+                ws[buf][lds_chunk(wr[i], wk[i] / 8 + s)] = __builtin_bit_cast(uint4, b[s]);
+        }
+    };
+
+    float4_t acc[NT][MT];
+#pragma unroll
+    for (int t = 0; t < NT; t++)
+#pragma unroll
+        for (int j = 0; j < MT; j++) acc[t][j] = float4_t{0.f, 0.f, 0.f, 0.f};
+
+#pragma unroll
+    for (int d = 0; d < PD; d++)
+        if (s0 + d < s1) load(d, s0 + d);
+    stash(0, 0);
+    if (s0 + PD < s1) load(0, s0 + PD);
+    __syncthreads();
+    for (int sb = s0; sb < s1; sb += PD) {
+#pragma unroll
+        for (int d = 0; d < PD; d++) {
+            const int st = sb + d;
+            if (st >= s1) break;
+            const int buf = (st - s0) & 1;
+#pragma unroll
+            for (int s = 0; s < 2; s++) {
+                half8_t xb[MT];
+#pragma unroll
+                for (int j = 0; j < MT; j++)
+                    xb[j] = __builtin_bit_cast(half8_t, xs[buf][lds_chunk((wm * MT + j) * 16 + c16, 2 * g + s)]);
+#pragma unroll
+                for (int t = 0; t < NT; t++) {
+                    const half8_t wa = __builtin_bit_cast(half8_t, ws[buf][lds_chunk((wn * NT + t) * 16 + c16, 2 * g + s)]);
+#pragma unroll
+                    for (int j = 0; j < MT; j++)
+                        acc[t][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wa, xb[j], acc[t][j], 0, 0, 0);
+                }
+            }
+            if (st + 1 < s1) {
+                const int dn = (d + 1) % PD;
+                stash(dn, buf ^ 1);
+                if (st + 1 + PD < s1) load(dn, st + 1 + PD);
+            }
+            __syncthreads();
+        }
+    }
+
+    // acc[t][j]: output columns 16 (wn NT + t) + 4g + i of row 16 (wm MT + j) + c16
+#pragma unroll
+    for (int j = 0; j < MT; j++) {
+        const int m = tm * BM + (wm * MT + j) * 16 + c16;
+        const bool mv = m < a.M;
+        if constexpr (EPI == LE_ROPE) {
+            float4_t v[NT];
+            const int col0 = tn * BN + wn * NT * 16;
+#pragma unroll
+            for (int t = 0; t < NT; t++) {
+                v[t] = acc[t][j];
+                if (a.scale) {
+                    const float4 sc = *reinterpret_cast<const float4*>(a.scale + min(col0 + 16 * t, a.N - 16) + 4 * g);
+                    v[t][0] *= sc.x; v[t][1] *= sc.y; v[t][2] *= sc.z; v[t][3] *= sc.w;
+                }
+            }
+            // the lanes of rows past M take part in the row sums; their table
+            // reads repeat the last row's
+            rope_store<HD, NT>(a, v, col0, mv ? m : a.M - 1, g, mv);
+        } else if constexpr (SWIGLU) {
+            const int F = a.N / 2;
+#pragma unroll
+            for (int t = 0; t < NT; t += 2) {
+                const int f = tn * (BN / 2) + (wn * NT + t) * 8 + 4 * g;
+                if (!mv || f >= F) continue;
+                float4 sg = make_float4(1.f, 1.f, 1.f, 1.f), su = sg;
+                if (a.scale) {
+                    sg = *reinterpret_cast<const float4*>(a.scale + f);
+                    su = *reinterpret_cast<const float4*>(a.scale + F + f);
+                }
+                const float4_t gt = acc[t][j], up = acc[t + 1][j];
+                uint2 o;
+                o.x = (uint32_t)f32_to_f16_bits(silu_mul(gt[0] * sg.x, up[0] * su.x)) |
+                      ((uint32_t)f32_to_f16_bits(silu_mul(gt[1] * sg.y, up[1] * su.y)) << 16);
+                o.y = (uint32_t)f32_to_f16_bits(silu_mul(gt[2] * sg.z, up[2] * su.z)) |
+                      ((uint32_t)f32_to_f16_bits(silu_mul(gt[3] * sg.w, up[3] * su.w)) << 16);
+                *reinterpret_cast<uint2*>(a.out16 + (size_t)m * F + f) = o;
+            }
+        } else {
+            float* orow = a.out + ((size_t)split * a.M + (mv ? m : 0)) * a.N;
+#pragma unroll
+            for (int t = 0; t < NT; t++) {
+                const int n = tn * BN + (wn * NT + t) * 16 + 4 * g;
+                if (!mv || n >= a.N) continue;
+                float4_t y = acc[t][j];
+                if (n + 4 <= a.N && a.N % 4 == 0) {
+                    if (EPI == LE_STORE && a.scale) {
+                        const float4 sc = *reinterpret_cast<const float4*>(a.scale + n);
+                        y[0] *= sc.x; y[1] *= sc.y; y[2] *= sc.z; y[3] *= sc.w;
+                    }
+                    *reinterpret_cast<float4*>(orow + n) = make_float4(y[0], y[1], y[2], y[3]);
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 4; i++)
+                        if (n + i < a.N) orow[n + i] = EPI == LE_STORE && a.scale ? y[i] * a.scale[n + i] : y[i];
+                }
+            }
+        }
+    }
+}
+
+// ---- attention ------------------------------------------------------------------
+//
+// Block = one KV head x 64 query rows (64/G consecutive positions x the G
+// heads of the group), 16 rows per wave; K/V tiles of 64 positions staged in
+// LDS (V transposed), the next tile in registers meanwhile.  S^T = K . Q^T,
+// so a lane holds scores of one query row and its running maximum and sum are
+// its own; P^T is then already the B operand of O^T = V^T . P^T (the k order
+// of that product is the order in which a lane holds its scores).
+//
+// Queries and probabilities are fp32: each goes in as the sum of two fp16
+// values (22 bits), the queries scaled per row so that neither part leaves the
+// fp16 range, the probabilities by 2^14.
+//
+// Infinities and NaN: scores that come out as NaN are recomputed in fp32 (an
+// infinite key times the two parts of a query may be inf - inf), and a V tile
+// that holds any takes the products of its own positions only, in fp32, so
+// that a position beyond a row's own never reaches that row.
+typedef unsigned short u16x2_t __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t max_exp(uint32_t m, uint4 v) {
+    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+        m = __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2_t, m),
+                                                                   __builtin_bit_cast(u16x2_t, w[i] & 0x7fff7fffu)));
+    return m;
+}
+__device__ __forceinline__ bool exp_nonfinite(uint32_t m) { return (m & 0xffffu) >= 0x7c00u || (m >> 16) >= 0x7c00u; }
+
+// fp32 as the sum of two fp16 values.
+__device__ __forceinline__ void split16(float v, _Float16& hi, _Float16& lo) {
+    hi = (_Float16)v;
+    lo = (_Float16)(v - (float)hi);
+}
+
+template <int HD, int G>
+__global__ __launch_bounds__(256, 2) void k_attn_long(int pos0, int M, const float* __restrict__ q,
+                                                      const uint16_t* __restrict__ kc,
+                                                      const uint16_t* __restrict__ vc, int nkv, int n_tb,
+                                                      uint16_t* __restrict__ out16) {
+    constexpr int TB = 64 / G;             // positions per block
+    constexpr int KB = HD == 256 ? 32 : 64;   // keys per tile (32: no spills at 256 dimensions)
+    constexpr int DS = HD / 32;            // k-steps of a score
+    constexpr int DT = HD / 16;            // 16-row tiles of O^T
+    constexpr int KS = HD / 8 + 1;         // uint4 per LDS row of K (16-byte pad)
+    constexpr int VS = KB / 8 + 1;         // uint4 per LDS row of V^T
+    constexpr int KU = KB * (HD / 8) / 256;        // K loads per thread
+    constexpr int VUN = (KB / 4) * (HD / 8);       // V units: 4 keys x 8 dims
+    constexpr int VU = (VUN + 255) / 256;
+    // the K tile, or the fp32 probabilities of a non-finite V tile (64 rows x KB)
+    __shared__ uint4 ks[KB * KS > 16 * KB ? KB * KS : 16 * KB];
+    __shared__ uint4 vs[HD * VS];
+
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int g = lane >> 4, c16 = lane & 15;
+    const int kvh = blockIdx.x % nkv;
+    const int t0 = (n_tb - 1 - blockIdx.x / nkv) * TB;   // the longest blocks first
+    const int nq = nkv * G, kvd = nkv * HD;
+    const int r = wave * 16 + c16;                       // this lane's query row
+    const int t = t0 + r / G, hq = kvh * G + r % G;
+    const bool tv = t < M;
+    const int L = pos0 + (tv ? t : M - 1) + 1;           // positions this row attends over
+    const int Lmax = pos0 + min(t0 + TB, M);             // and the block
+    const float* qrow = q + ((size_t)(tv ? t : M - 1) * nq + hq) * HD;
+
+    // K/V tile loads of this thread
+    const uint16_t* kp = kc + (size_t)kvh * HD;
+    const uint16_t* vp = vc + (size_t)kvh * HD;
+    uint4 kr[KU], vr[VU][4];
+    auto load = [&](int p0) {
+#pragma unroll
+        for (int i = 0; i < KU; i++) {
+            const int u = tid + 256 * i, key = u / (HD / 8), ch = u % (HD / 8);
+            kr[i] = p0 + key < Lmax ? *reinterpret_cast<const uint4*>(kp + (size_t)(p0 + key) * kvd + 8 * ch)
+                                    : make_uint4(0u, 0u, 0u, 0u);
+        }
+#pragma unroll
+        for (int i = 0; i < VU; i++) {
+            const int u = tid + 256 * i, kg = u % (KB / 4), db = u / (KB / 4);
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                vr[i][j] = db < HD / 8 && p0 + 4 * kg + j < Lmax
+                               ? *reinterpret_cast<const uint4*>(vp + (size_t)(p0 + 4 * kg + j) * kvd + 8 * db)
+                               : make_uint4(0u, 0u, 0u, 0u);
+        }
+    };
+    load(0);
+
+    // the query row as fp16 pairs, scaled by 2^e to a maximum in [2^14, 2^15)
+    half8_t qh[DS], ql[DS];
+    float qscale;
+    {
+        float qv[DS][8], mx = 0.0f;
+#pragma unroll
+        for (int s = 0; s < DS; s++) {
+            const float4 lo = *reinterpret_cast<const float4*>(qrow + 32 * s + 8 * g);
+            const float4 hi = *reinterpret_cast<const float4*>(qrow + 32 * s + 8 * g + 4);
+            qv[s][0] = lo.x; qv[s][1] = lo.y; qv[s][2] = lo.z; qv[s][3] = lo.w;
+            qv[s][4] = hi.x; qv[s][5] = hi.y; qv[s][6] = hi.z; qv[s][7] = hi.w;
+#pragma unroll
+            for (int e = 0; e < 8; e++) mx = fmaxf(mx, fabsf(qv[s][e]));
+        }
+        mx = rows_max4(mx);
+        int ex = 0;
+        if (mx > 0.0f && mx < INFINITY) {
+            ex = 14 - ilogbf(mx);
+            ex = ex > 100 ? 100 : ex;
+        }
+        const float up = ldexpf(1.0f, ex);
+        qscale = ldexpf(1.0f / sqrtf((float)HD), -ex);
+#pragma unroll
+        for (int s = 0; s < DS; s++)
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                _Float16 h, l;
+                split16(qv[s][e] * up, h, l);
+                qh[s][e] = h;
+                ql[s][e] = l;
+            }
+    }
+
+    float4_t o[DT];
+#pragma unroll
+    for (int d = 0; d < DT; d++) o[d] = float4_t{0.f, 0.f, 0.f, 0.f};
+    float runM = -INFINITY, runL = 0.0f;
+
+    for (int p0 = 0; p0 < Lmax; p0 += KB) {
+        uint32_t vmax = 0;
+#pragma unroll
+        for (int i = 0; i < KU; i++) {
+            const int u = tid + 256 * i;
+            ks[(u / (HD / 8)) * KS + u % (HD / 8)] = kr[i];
+        }
+#pragma unroll
+        for (int i = 0; i < VU; i++) {
+            const int u = tid + 256 * i, kg = u % (KB / 4), db = u / (KB / 4);
+            if (VUN % 256 != 0 && db >= HD / 8) break;
+            // key 4 kg + j lies at offset 32 (kg/8) + 8 (kg%4) + 4 (kg/4 % 2) + j of
+            // its row: the order of the second product
+            const int off = 32 * (kg >> 3) + 8 * (kg & 3) + 4 * ((kg >> 2) & 1);
+            uint32_t wd[4][4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                vmax = max_exp(vmax, vr[i][j]);
+                wd[j][0] = vr[i][j].x; wd[j][1] = vr[i][j].y; wd[j][2] = vr[i][j].z; wd[j][3] = vr[i][j].w;
+            }
+            uint16_t* vb = reinterpret_cast<uint16_t*>(vs) + off;
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                const uint32_t sel = (e & 1) ? 0x07060302u : 0x05040100u;
+                uint2 w2;
+                w2.x = __builtin_amdgcn_perm(wd[1][e / 2], wd[0][e / 2], sel);
+                w2.y = __builtin_amdgcn_perm(wd[3][e / 2], wd[2][e / 2], sel);
+                *reinterpret_cast<uint2*>(vb + (8 * db + e) * (VS * 8)) = w2;
+            }
+        }
+        const bool slow = __syncthreads_or(exp_nonfinite(vmax));
+        if (p0 + KB < Lmax) load(p0 + KB);
+
+        // scores: s[kt][i] = key p0 + 16 kt + 4 g + i, then their exponentials
+        float4_t s[KB / 16];
+        float alpha, ls, mx;
+        auto softmax = [&]() {
+            if (p0 + KB > pos0 + t0 + 1) {      // some row of the block ends inside this tile
+#pragma unroll
+                for (int kt = 0; kt < KB / 16; kt++)
+#pragma unroll
+                    for (int i = 0; i < 4; i++)
+                        if (p0 + 16 * kt + 4 * g + i >= L) s[kt][i] = -INFINITY;
+            }
+            mx = -INFINITY;
+#pragma unroll
+            for (int kt = 0; kt < KB / 16; kt++)
+                mx = fmaxf(mx, fmaxf(fmaxf(s[kt][0], s[kt][1]), fmaxf(s[kt][2], s[kt][3])));
+            mx = fmaxf(runM, rows_max4(mx));
+            const float ref = mx == -INFINITY ? 0.0f : mx;   // no score above -inf yet: p = 0
+            alpha = expf(runM - ref);
+            ls = 0.0f;
+#pragma unroll
+            for (int kt = 0; kt < KB / 16; kt++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    s[kt][i] = expf(s[kt][i] - ref);
+                    ls = ls + s[kt][i];
+                }
+        };
+#pragma unroll
+        for (int kt = 0; kt < KB / 16; kt++) {
+            s[kt] = float4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int d = 0; d < DS; d++) {
+                const half8_t k8 = __builtin_bit_cast(half8_t, ks[(16 * kt + c16) * KS + 4 * d + g]);
+                s[kt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(k8, qh[d], s[kt], 0, 0, 0);
+                s[kt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(k8, ql[d], s[kt], 0, 0, 0);
+            }
+#pragma unroll
+            for (int i = 0; i < 4; i++) s[kt][i] = s[kt][i] * qscale;
+        }
+        softmax();
+        if (__any(ls != ls)) {
+            const uint16_t* kb = reinterpret_cast<const uint16_t*>(ks);
+            const float sc = 1.0f / sqrtf((float)HD);
+#pragma unroll
+            for (int kt = 0; kt < KB / 16; kt++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const uint16_t* kk = kb + (16 * kt + 4 * g + i) * (KS * 8);
+                    float sum = 0.0f;
+#pragma unroll 1
+                    for (int d = 0; d < HD; d++) sum = sum + qrow[d] * f16_bits_to_f32(kk[d]);
+                    s[kt][i] = sum * sc;
+                }
+            softmax();
+        }
+        runM = mx;
+        runL = runL * alpha + ls;
+#pragma unroll
+        for (int d = 0; d < DT; d++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) o[d][i] = o[d][i] * alpha;
+        if (!slow) {
+#pragma unroll
+            for (int pr = 0; pr < KB / 32; pr++) {
+                half8_t ph, pl;
+#pragma unroll
+                for (int e = 0; e < 8; e++) {
+                    _Float16 h, l;
+                    split16(s[2 * pr + e / 4][e % 4] * 16384.0f, h, l);
+                    ph[e] = h;
+                    pl[e] = l;
+                }
+#pragma unroll
+                for (int d = 0; d < DT; d++) {
+                    const half8_t v8 = __builtin_bit_cast(half8_t, vs[(16 * d + c16) * VS + 4 * pr + g]);
+                    o[d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(v8, ph, o[d], 0, 0, 0);
+                    o[d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(v8, pl, o[d], 0, 0, 0);
+                }
+            }
+        } else {
+            __syncthreads();                // every wave is done with the K tile
+            float* pf = reinterpret_cast<float*>(ks) + (size_t)wave * 16 * KB;   // [16 rows][KB]
+#pragma unroll
+            for (int kt = 0; kt < KB / 16; kt++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) pf[c16 * KB + 16 * kt + 4 * g + i] = s[kt][i];
+            __syncthreads();
+            const uint16_t* vb = reinterpret_cast<const uint16_t*>(vs);
+#pragma unroll 1
+            for (int key = 0; key < KB; key++) {
+                if (p0 + key >= L) break;
+                const float p = pf[c16 * KB + key] * 16384.0f;
+                const int off = 32 * (key >> 5) + 8 * ((key >> 2) & 3) + 4 * ((key >> 4) & 1) + (key & 3);
+#pragma unroll
+                for (int d = 0; d < DT; d++)
+#pragma unroll
+                    for (int i = 0; i < 4; i++)
+                        o[d][i] = o[d][i] + p * f16_bits_to_f32(vb[(16 * d + 4 * g + i) * (VS * 8) + off]);
+            }
+        }
+        __syncthreads();                    // the tile is rewritten
+    }
+    if (!tv) return;
+    const float l = rows_sum4(runL) * 16384.0f;
+    uint16_t* dst = out16 + ((size_t)t * nq + hq) * HD + 4 * g;
+#pragma unroll
+    for (int d = 0; d < DT; d++) {
+        uint2 w;
+        w.x = (uint32_t)f32_to_f16_bits(o[d][0] / l) | ((uint32_t)f32_to_f16_bits(o[d][1] / l) << 16);
+        w.y = (uint32_t)f32_to_f16_bits(o[d][2] / l) | ((uint32_t)f32_to_f16_bits(o[d][3] / l) << 16);
+        *reinterpret_cast<uint2*>(dst + 16 * d) = w;
+    }
+}
+
+// ---- tile choice ------------------------------------------------------------------
+
+struct LongTile {
+    int bm, bn, splits;
+};
+
+int cdiv(int a, int b) { return (a + b - 1) / b; }
+
+// Tiles of 128 x 128 once they fill the chip twice over, else 64-row or 64 x 64
+// ones; the residual projections (which can sum partials) also split K into
+// runs of at least 256 until there are about 512 blocks.
+LongTile long_tile(int M, int N, int K, bool can_split, bool wide) {
+    LongTile t;
+    t.splits = 1;
+    if (cdiv(M, 128) * cdiv(N, 128) >= 256) t.bm = t.bn = 128;
+    else if (wide) t.bm = 64, t.bn = 128;
+    else t.bm = t.bn = 64;
+    if (can_split) {
+        const int tiles = cdiv(M, t.bm) * cdiv(N, t.bn), nst = cdiv(K, kKT);
+        int ns = 512 / tiles;
+        if (ns > K / 256) ns = K / 256;
+        if (ns > 8) ns = 8;
+        if (ns < 1) ns = 1;
+        const int per = cdiv(nst, ns);
+        t.splits = cdiv(nst, per);          // none is empty
+    }
+    return t;
+}
+
+template <int KIND, int EPI, int HD>
+int long_launch_kind(const LongArgs& a, const LongTile& t, hipStream_t s) {
+    dim3 grid((unsigned)(a.tiles_m * a.tiles_n * a.splits)), block(256);
+    if constexpr (EPI == LE_ROPE) {
+        if (t.bm == 128) hipLaunchKernelGGL((k_long_gemm<KIND, 128, 128, 1, 1, EPI, HD>), grid, block, 0, s, a);
+        else hipLaunchKernelGGL((k_long_gemm<KIND, 64, 128, 1, 2, EPI, HD>), grid, block, 0, s, a);
+    } else {
+        if (t.bm == 128) hipLaunchKernelGGL((k_long_gemm<KIND, 128, 128, 2, 1, EPI, 0>), grid, block, 0, s, a);
+        else hipLaunchKernelGGL((k_long_gemm<KIND, 64, 64, 2, 2, EPI, 0>), grid, block, 0, s, a);
+    }
+    return hipGetLastError() == hipSuccess ? 0 : -4;
+}
+
+template <int EPI, int HD>
+int long_launch(LongArgs& a, int kind, const LongTile& t, void* stream) {
+    a.tiles_m = cdiv(a.M, t.bm);
+    a.tiles_n = EPI == LE_SWIGLU ? cdiv(a.N / 2, t.bn / 2) : cdiv(a.N, t.bn);
+    a.splits = t.splits;
+    a.per_split = cdiv(cdiv(a.K, kKT), t.splits);
+    if ((long long)a.tiles_m * a.tiles_n * a.splits > 0x7fffffffLL) return -1;
+    hipStream_t s = (hipStream_t)stream;
+    switch (kind) {
+        case MDX_W_F16: return long_launch_kind<MDX_W_F16, EPI, HD>(a, t, s);
+        case MDX_W_I8: return long_launch_kind<MDX_W_I8, EPI, HD>(a, t, s);
+        case MDX_W_I4: return long_launch_kind<MDX_W_I4, EPI, HD>(a, t, s);
+        default: return -5;
+    }
+}
+
+LongArgs long_args(const uint16_t* x16, int M, const mdx_wdesc* w) {
+    LongArgs a = {};
+    a.x16 = x16;
+    a.w = (const uint8_t*)w->w;
+    a.scale = w->scale;
+    a.M = M;
+    a.K = w->K;
+    a.N = w->N;
+    return a;
+}
+
+}  // namespace
+
+extern "C" {
+
+int mdx_long_ok(const mdx_wdesc* w) {
+    return w->kind >= MDX_W_F16 && w->kind <= MDX_W_I4 && w->K > 0 && w->K % 32 == 0 && w->N > 0;
+}
+
+int mdx_launch_long_gemm(const uint16_t* x16, int M, const mdx_wdesc* w, int swiglu, void* out, void* stream) {
+    if (M <= 0 || !out || !mdx_long_ok(w) || (swiglu && w->N % 8)) return -1;
+    LongArgs a = long_args(x16, M, w);
+    const LongTile t = long_tile(M, w->N, w->K, false, false);
+    if (swiglu) {
+        a.out16 = (uint16_t*)out;
+        return long_launch<LE_SWIGLU, 0>(a, w->kind, t, stream);
+    }
+    a.out = (float*)out;
+    return long_launch<LE_STORE, 0>(a, w->kind, t, stream);
+}
+
+size_t mdx_long_scratch_floats(int M, int N) {
+    /* splits <= min(8, 512 / tiles), each tile at most 128 x 128 */
+    const size_t mn = (size_t)M * N, cap = (size_t)512 * 128 * 128;
+    const size_t most = 8 * mn < cap ? 8 * mn : cap;
+    return mn > most ? mn : most;
+}
+
+int mdx_launch_long_residual_norm(const uint16_t* x16, int M, const mdx_wdesc* w, float* hidden,
+                                  const float* norm_w, float eps, uint16_t* x16_out, float* scratch,
+                                  void* stream) {
+    if (M <= 0 || !mdx_long_ok(w) || w->N % 4) return -1;
+    LongArgs a = long_args(x16, M, w);
+    const LongTile t = long_tile(M, w->N, w->K, true, false);
+    a.out = scratch;
+    const int rc = long_launch<LE_PART, 0>(a, w->kind, t, stream);
+    return rc ? rc : mdx_launch_residual_norm(scratch, t.splits, M, M, w->N, w->scale, hidden, norm_w, eps,
+                                              x16_out, stream);
+}
+
+int mdx_launch_long_qkv_rope(const uint16_t* x16, int M, const mdx_wdesc* w, int pos0, const float* q_norm,
+                             const float* k_norm, float eps, const float* cos_t, const float* sin_t, int nq,
+                             int nkv, int hd, int rope_style, float* q_out, uint16_t* k_cache,
+                             uint16_t* v_cache, void* stream) {
+    if (M <= 0 || pos0 < 0 || !mdx_long_ok(w) || w->N != (nq + 2 * nkv) * hd) return -1;
+    LongArgs a = long_args(x16, M, w);
+    a.pos0 = pos0;
+    a.nq = nq;
+    a.nkv = nkv;
+    a.style = rope_style;
+    a.q_norm = q_norm;
+    a.k_norm = k_norm;
+    a.eps = eps;
+    a.cos_t = cos_t;
+    a.sin_t = sin_t;
+    a.q_out = q_out;
+    a.kc = k_cache;
+    a.vc = v_cache;
+    const LongTile t = long_tile(M, w->N, w->K, false, true);
+    if (hd == 64) return long_launch<LE_ROPE, 64>(a, w->kind, t, stream);
+    if (hd == 128) return long_launch<LE_ROPE, 128>(a, w->kind, t, stream);
+    return -5;
+}
+
+int mdx_launch_long_attn(int pos0, const float* q, int M, const uint16_t* k_cache, const uint16_t* v_cache,
+                         int nq, int nkv, int hd, uint16_t* out16, void* stream) {
+    if (nkv <= 0 || nq % nkv || M <= 0 || pos0 < 0) return -1;
+    const int G = nq / nkv;
+    if (G < 1 || G > 4 || (G & (G - 1))) return -5;
+    const int n_tb = cdiv(M, 64 / G);
+    dim3 grid((unsigned)(n_tb * nkv));
+#define MDX_LATTN(HD_, G_)                                                                                 \
+    if (hd == HD_ && G == G_) {                                                                            \
+        hipLaunchKernelGGL((k_attn_long<HD_, G_>), grid, dim3(256), 0, (hipStream_t)stream, pos0, M, q,    \
+                           k_cache, v_cache, nkv, n_tb, out16);                                            \
+        return hipGetLastError() == hipSuccess ? 0 : -4;                                                   \
+    }
+    MDX_LATTN(64, 1) MDX_LATTN(64, 2) MDX_LATTN(64, 4)
+    MDX_LATTN(128, 1) MDX_LATTN(128, 2) MDX_LATTN(128, 4)
+    MDX_LATTN(256, 1) MDX_LATTN(256, 2) MDX_LATTN(256, 4)
+#undef MDX_LATTN
+    return -5;
+}
+
+}  // extern "C"

@@ -146,6 +146,11 @@ def lib() -> C.CDLL:
             "mdx_device_synchronize": (C.c_int, []),
             "mdx_debug_gemv": (C.c_int, [C.c_int, C.c_int, C.c_int, P, _F, _F, _F]),
             "mdx_debug_gemm": (C.c_int, [C.c_int, C.c_int, C.c_int, C.c_int, P, _F, _F, _F]),
+            "mdx_debug_long_gemm": (C.c_int, [C.c_int, C.c_int, C.c_int, C.c_int, P, _F, _F, _F]),
+            "mdx_debug_long_residual": (C.c_int, [C.c_int, C.c_int, C.c_int, C.c_int, P, _F, _F, _F,
+                                                  _F, C.c_float, C.POINTER(C.c_uint16)]),
+            "mdx_debug_long_attn": (C.c_int, [C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, _F, _U16,
+                                              _U16, _F]),
             "mdx_debug_gemm_splits": (C.c_int, [C.c_int, C.c_int, C.c_int, _I]),
             "mdx_debug_persist_kv_rows": (C.c_longlong, [C.c_int, C.c_int, C.POINTER(C.c_longlong)]),
             "mdx_debug_gemm_residual": (C.c_int, [C.c_int, C.c_int, C.c_int, C.c_int, P, _F, _F, _F,
@@ -260,27 +265,26 @@ def gemv(kind: int, K: int, N: int, w: np.ndarray, scales, x) -> np.ndarray:
     return y
 
 
-def gemm(kind: int, M: int, K: int, N: int, w: np.ndarray, scales, x) -> np.ndarray:
+def gemm(kind: int, M: int, K: int, N: int, w: np.ndarray, scales, x, long: bool = False) -> np.ndarray:
     w = np.ascontiguousarray(w)
     y = np.empty(M * N, np.float32)
     s, x = _f32(scales), _f32(x)
-    _check(lib().mdx_debug_gemm(kind, M, K, N, w.ctypes.data, _p(s, _F), _p(x, _F), _p(y, _F)),
-           "gemm")
+    fn = lib().mdx_debug_long_gemm if long else lib().mdx_debug_gemm
+    _check(fn(kind, M, K, N, w.ctypes.data, _p(s, _F), _p(x, _F), _p(y, _F)), "gemm")
     return y.reshape(M, N)
 
 
 def gemm_residual(kind: int, M: int, K: int, N: int, w: np.ndarray, scales, x, hidden, norm_w,
-                  eps: float = 1e-6):
+                  eps: float = 1e-6, long: bool = False):
     """Prefill residual projection: (hidden + fp16(x) . W * scale, fp16 normed rows or None)."""
     w = np.ascontiguousarray(w)
     s, x = _f32(scales), _f32(x)
     h = np.array(_f32(hidden), dtype=np.float32, copy=True).reshape(M, N)
     nw = _f32(norm_w)
     out = np.zeros((M, N), np.uint16) if norm_w is not None else None
-    _check(lib().mdx_debug_gemm_residual(kind, M, K, N, w.ctypes.data, _p(s, _F), _p(x, _F),
-                                         _p(h, _F), _p(nw, _F), eps,
-                                         out.ctypes.data_as(C.POINTER(C.c_uint16)) if out is not None
-                                         else None), "gemm_residual")
+    fn = lib().mdx_debug_long_residual if long else lib().mdx_debug_gemm_residual
+    _check(fn(kind, M, K, N, w.ctypes.data, _p(s, _F), _p(x, _F), _p(h, _F), _p(nw, _F), eps,
+              out.ctypes.data_as(C.POINTER(C.c_uint16)) if out is not None else None), "gemm_residual")
     return h, out
 
 
@@ -299,13 +303,13 @@ def attn_decode(nq, nkv, hd, pos, style, theta, eps, q_norm, k_norm, qkv, k16, v
     return out, kn16, vn16
 
 
-def attn_prefill(nq, nkv, hd, S, M, q, k16, v16) -> np.ndarray:
+def attn_prefill(nq, nkv, hd, S, M, q, k16, v16, long: bool = False) -> np.ndarray:
     q = _f32(q)
     k16 = np.ascontiguousarray(k16, np.uint16)
     v16 = np.ascontiguousarray(v16, np.uint16)
     out = np.empty(M * nq * hd, np.float32)
-    _check(lib().mdx_debug_attn_prefill(nq, nkv, hd, S, M, _p(q, _F), _p(k16, _U16), _p(v16, _U16),
-                                        _p(out, _F)), "attn_prefill")
+    fn = lib().mdx_debug_long_attn if long else lib().mdx_debug_attn_prefill
+    _check(fn(nq, nkv, hd, S, M, _p(q, _F), _p(k16, _U16), _p(v16, _U16), _p(out, _F)), "attn_prefill")
     return out.reshape(M, nq * hd)
 
 
