@@ -55,10 +55,24 @@ struct GemvArgs {
     float* hidden_out;
     // EP_LOGITS: fused argmax and step bookkeeping
     mdx_state* st;
-    unsigned long long* amax_key;
-    unsigned int* done;
+    void* lm_scr;         // LmScratch
     int* out_tokens;
     int advance;
+};
+
+// What the lm_head kernels share between workgroups, zero between launches
+// except for the keys.  Arrival is counted per group of workgroups, each
+// counter on a line of its own, and the last of a group counts at the top: one
+// address that every workgroup of a launch updates serialises them (two such
+// atomics per workgroup before: 100 rows + 32 tokens of a model with an
+// 8000 x 512 int8 head 8.59 -> 7.80 ms, 25 us a token; 16 steps with a
+// 2048 x 1024 fp32 head 1.70 -> 1.56 ms).
+constexpr int kLmBlocks = 256;       // k_lmhead_i8_1k
+constexpr int kLmMaxBlocks = 1024;   // k_gemv
+constexpr int kLmGroups = 32;
+struct LmScratch {
+    struct { unsigned n, pad[31]; } cnt[kLmGroups + 1];   // [kLmGroups]: the top
+    unsigned long long keys[kLmMaxBlocks];
 };
 
 template <int KIND> struct KindTraits;
@@ -314,6 +328,70 @@ __device__ __forceinline__ void store_rows(const GemvArgs& a, const RowSet<KIND,
     }
 }
 
+__device__ __forceinline__ unsigned long long wave_max_key(unsigned long long best) {
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const unsigned lo = __shfl_xor((unsigned)(best & 0xffffffffull), off, 64);
+        const unsigned hi = __shfl_xor((unsigned)(best >> 32), off, 64);
+        const unsigned long long k = ((unsigned long long)hi << 32) | lo;
+        best = k > best ? k : best;
+    }
+    return best;
+}
+
+// The end of an lm_head launch: the workgroup's argmax key from its waves'
+// (best: wave-uniform), and, in the last workgroup to arrive, the argmax of
+// all keys and the step's bookkeeping.
+__device__ __forceinline__ void lm_finish(const GemvArgs& a, unsigned long long best, unsigned long long* bkey,
+                                          int* last_block) {
+    LmScratch* scr = reinterpret_cast<LmScratch*>(a.lm_scr);
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    if (lane == 0) bkey[wave] = best;
+    __syncthreads();
+    const int n_grp = min(kLmGroups, (int)gridDim.x);
+    if (tid == 0) {
+        unsigned long long bk = bkey[0];
+        for (int w = 1; w < 4; w++) bk = bkey[w] > bk ? bkey[w] : bk;
+        // the key goes out with a device-scope store that completes before
+        // the arrival is counted, and the last block reads the keys with
+        // device-scope loads: no cache write-back or invalidate is needed
+        __hip_atomic_store(&scr->keys[blockIdx.x], bk, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __builtin_amdgcn_s_waitcnt(0);
+        const int grp = blockIdx.x % n_grp;
+        const unsigned in_grp = (gridDim.x - grp + n_grp - 1) / n_grp;
+        int last = 0;
+        if (__hip_atomic_fetch_add(&scr->cnt[grp].n, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == in_grp - 1)
+            last = __hip_atomic_fetch_add(&scr->cnt[kLmGroups].n, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
+                   (unsigned)n_grp - 1;
+        *last_block = last;
+    }
+    __syncthreads();
+    if (!*last_block) return;
+    unsigned long long k = 0ull;
+    for (int i = tid; i < (int)gridDim.x; i += 256) {
+        const unsigned long long v = __hip_atomic_load(&scr->keys[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        k = v > k ? v : k;
+    }
+    k = wave_max_key(k);
+    if (lane == 0) bkey[wave] = k;
+    __syncthreads();
+    if (tid <= kLmGroups) __hip_atomic_store(&scr->cnt[tid].n, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (tid == 0) {
+        k = bkey[0];
+        for (int w = 1; w < 4; w++) k = bkey[w] > k ? bkey[w] : k;
+        const int tok = ref_argmax_index(k);
+        mdx_state* st = a.st;
+        st->argmax = tok;
+        st->token = tok;
+        st->mode = 0;
+        if (a.out_tokens) {
+            a.out_tokens[st->n_out] = tok;
+            st->n_out = st->n_out + 1;
+        }
+        st->pos = st->pos + a.advance;
+    }
+}
+
 // The GEMV.  Blocks of 256 threads (4 waves x RW rows) walk the row blocks
 // with a grid stride; the next row block's weights are requested before the
 // current one is reduced.
@@ -383,35 +461,7 @@ __global__ __launch_bounds__(256) void k_gemv(GemvArgs a) {
         if (!single && nb < nblk) rs.load(a, row_bytes, nchunks, 0, lane, wv);
     }
 
-    if (a.epi == EP_LOGITS) {
-        if (lane == 0) bkey[wave] = best;
-        __syncthreads();
-        if (tid == 0) {
-            unsigned long long b = bkey[0];
-            for (int w = 1; w < 4; w++) b = bkey[w] > b ? bkey[w] : b;
-            // device-scope atomics throughout, the maximum completed before
-            // the arrival is counted: no cache write-back is needed
-            if (b) __hip_atomic_fetch_max(a.amax_key, b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __builtin_amdgcn_s_waitcnt(0);
-            const unsigned prev = __hip_atomic_fetch_add(a.done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            last_block = prev == gridDim.x - 1;
-        }
-        __syncthreads();
-        if (last_block && tid == 0) {
-            const unsigned long long k = atomicExch(a.amax_key, 0ull);
-            atomicExch(a.done, 0u);
-            const int tok = ref_argmax_index(k);
-            mdx_state* st = a.st;
-            st->argmax = tok;
-            st->token = tok;
-            st->mode = 0;
-            if (a.out_tokens) {
-                a.out_tokens[st->n_out] = tok;
-                st->n_out = st->n_out + 1;
-            }
-            st->pos = st->pos + a.advance;
-        }
-    }
+    if (a.epi == EP_LOGITS) lm_finish(a, best, bkey, &last_block);
 }
 
 // The GEMV when every workgroup takes exactly one row block and a lane's
@@ -458,12 +508,8 @@ __global__ __launch_bounds__(256) void k_gemv_once(GemvArgs a) {
 // block b streams rows [b*N/grid, (b+1)*N/grid); each wave takes batches of
 // 16 rows, 4 batches apart, with three batches in registers (two in flight
 // while one is multiplied).  x = fp16(RMSNorm(hidden)).  Each block stores its
-// argmax key; arrival is counted in 8 group counters (so no single address
-// takes all the atomics) and the last block reduces the keys and does the
-// step bookkeeping of k_gemv's EP_LOGITS.
+// argmax key (lm_finish).
 constexpr int kLmRows = 16;
-constexpr int kLmBlocks = 256;
-constexpr int kLmGroups = 8;
 __global__ __launch_bounds__(256) void k_lmhead_i8_1k(GemvArgs a) {
     constexpr int U = kLmRows;
     constexpr int PER = 64 / U;
@@ -514,67 +560,7 @@ __global__ __launch_bounds__(256) void k_lmhead_i8_1k(GemvArgs a) {
         if (base + 16 * U < re) load(w1, sc1, base + 16 * U);
         consume(w2, sc2, base + 8 * U);
     }
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        const unsigned lo = __shfl_xor((unsigned)(best & 0xffffffffull), off, 64);
-        const unsigned hi = __shfl_xor((unsigned)(best >> 32), off, 64);
-        const unsigned long long k = ((unsigned long long)hi << 32) | lo;
-        best = k > best ? k : best;
-    }
-    if (lane == 0) bkey[wave] = best;
-    __syncthreads();
-    // scratch: [16, 48) group counters, [48, 52) group-done counter, [64, ...) keys
-    unsigned* cnt = reinterpret_cast<unsigned*>(reinterpret_cast<char*>(a.amax_key) + 16);
-    unsigned* top = reinterpret_cast<unsigned*>(reinterpret_cast<char*>(a.amax_key) + 48);
-    unsigned long long* keys = reinterpret_cast<unsigned long long*>(reinterpret_cast<char*>(a.amax_key) + 64);
-    if (tid == 0) {
-        unsigned long long bk = bkey[0];
-        for (int w = 1; w < 4; w++) bk = bkey[w] > bk ? bkey[w] : bk;
-        // the key goes out with a device-scope store that completes before
-        // the arrival is counted, and the last block reads the keys with
-        // device-scope loads: no cache write-back or invalidate is needed
-        __hip_atomic_store(&keys[blockIdx.x], bk, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __builtin_amdgcn_s_waitcnt(0);
-        const int grp = blockIdx.x % kLmGroups;
-        const unsigned in_grp = (gridDim.x - grp + kLmGroups - 1) / kLmGroups;
-        int last = 0;
-        if (__hip_atomic_fetch_add(&cnt[grp], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == in_grp - 1)
-            last = __hip_atomic_fetch_add(top, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == kLmGroups - 1;
-        last_block = last;
-    }
-    __syncthreads();
-    if (last_block) {
-        unsigned long long k = 0ull;
-        for (int i = tid; i < (int)gridDim.x; i += 256) {
-            const unsigned long long v = __hip_atomic_load(&keys[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            k = v > k ? v : k;
-        }
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-            const unsigned lo = __shfl_xor((unsigned)(k & 0xffffffffull), off, 64);
-            const unsigned hi = __shfl_xor((unsigned)(k >> 32), off, 64);
-            const unsigned long long k2 = ((unsigned long long)hi << 32) | lo;
-            k = k2 > k ? k2 : k;
-        }
-        if (lane == 0) bkey[wave] = k;
-        __syncthreads();
-        if (tid < kLmGroups) __hip_atomic_store(&cnt[tid], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    if (last_block && tid == 0) {
-        unsigned long long k = bkey[0];
-        for (int w = 1; w < 4; w++) k = bkey[w] > k ? bkey[w] : k;
-        __hip_atomic_store(top, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const int tok = ref_argmax_index(k);
-        mdx_state* st = a.st;
-        st->argmax = tok;
-        st->token = tok;
-        st->mode = 0;
-        if (a.out_tokens) {
-            a.out_tokens[st->n_out] = tok;
-            st->n_out = st->n_out + 1;
-        }
-        st->pos = st->pos + a.advance;
-    }
+    lm_finish(a, wave_max_key(best), bkey, &last_block);
 }
 
 typedef void (*GemvKernel)(GemvArgs);
@@ -1134,7 +1120,7 @@ int mdx_launch_gemv(const float* x, const mdx_wdesc* w, int x_fp32_exact, float*
     return launch_gemv(kind, a, rows_per_wave_for(a.N), 0, stream);
 }
 
-size_t mdx_lmhead_scratch_bytes(void) { return 64 + 8 * kLmBlocks; }
+size_t mdx_lmhead_scratch_bytes(void) { return sizeof(LmScratch); }
 
 int mdx_launch_lmhead(const float* hidden, const float* norm_w, float eps, const mdx_wdesc* w,
                       float* logits, void* scratch, mdx_state* state, int* out_tokens, int advance,
@@ -1146,8 +1132,7 @@ int mdx_launch_lmhead(const float* hidden, const float* norm_w, float eps, const
     a.eps = eps;
     a.epi = EP_LOGITS;
     a.out_f32 = logits;
-    a.amax_key = (unsigned long long*)scratch;
-    a.done = (unsigned int*)((char*)scratch + 8);
+    a.lm_scr = scratch;
     a.st = state;
     a.out_tokens = out_tokens;
     a.advance = advance;
@@ -1157,7 +1142,7 @@ int mdx_launch_lmhead(const float* hidden, const float* norm_w, float eps, const
         hipLaunchKernelGGL(k_lmhead_i8_1k, dim3(kLmBlocks), dim3(256), 0, (hipStream_t)stream, a);
         return hipGetLastError() == hipSuccess ? 0 : -4;
     }
-    return launch_gemv(kind, a, rows_per_wave_for(w->N), 1024, stream);
+    return launch_gemv(kind, a, rows_per_wave_for(w->N), kLmMaxBlocks, stream);
 }
 
 int mdx_launch_advance(mdx_state* state, int advance, void* stream) {
