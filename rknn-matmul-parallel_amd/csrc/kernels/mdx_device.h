@@ -70,6 +70,14 @@ int mdxrt_event_create(void** ev);
 int mdxrt_event_destroy(void* ev);
 int mdxrt_event_record(void* ev, void* stream);
 int mdxrt_event_elapsed_ms(void* start, void* stop, float* ms);
+/* Copy by a kernel between device memory and pinned host memory (16-byte
+ * addresses and size). */
+int mdxrt_copy16(void* dst, const void* src, size_t bytes, void* stream);
+/* mdxrt_signal stores 1 in the pinned word *flag once everything before it on
+ * the stream is complete; mdxrt_wait returns when it is there.  The caller
+ * clears the word before it issues the work. */
+int mdxrt_signal(int* flag, void* stream);
+int mdxrt_wait(int* flag, void* stream);
 /* Fill `n` 32-bit words with `value` on the stream (a kernel, never a
  * memset node, so it is safe inside captured graphs). */
 int mdxrt_fill_u32(void* dst, uint32_t value, size_t n, void* stream);

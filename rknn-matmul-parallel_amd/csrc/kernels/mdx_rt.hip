@@ -3,6 +3,7 @@
 // last HIP message is kept for diagnostics.
 #include <hip/hip_runtime.h>
 
+#include <chrono>
 #include <cstdio>
 #include <cstring>
 #include <mutex>
@@ -29,6 +30,20 @@ __global__ void k_fill_u32(uint32_t* dst, uint32_t value, size_t n) {
     size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     size_t stride = (size_t)gridDim.x * blockDim.x;
     for (; i < n; i += stride) dst[i] = value;
+}
+
+// 16-byte words from mapped host memory to device memory (or back).  A copy of
+// a few MB by a kernel runs at the bus rate like the runtime's (3 MB 73 us,
+// 8 MB 163 us), without the ~10 us that a small asynchronous copy waits.
+__global__ __launch_bounds__(256) void k_copy16(uint4* dst, const uint4* src, size_t n) {
+    const size_t stride = (size_t)gridDim.x * blockDim.x;
+    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) dst[i] = src[i];
+}
+
+// The word the host polls (mdxrt_wait): everything before this kernel on its
+// stream is complete, its stores to host memory included.
+__global__ void k_signal(int* flag) {
+    if (threadIdx.x == 0) __hip_atomic_store(flag, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 }  // namespace
@@ -242,6 +257,41 @@ int mdxrt_event_elapsed_ms(void* start, void* stop, float* ms) {
     MDX_CHECK(hipEventSynchronize((hipEvent_t)stop), "hipEventSynchronize");
     MDX_CHECK(hipEventElapsedTime(ms, (hipEvent_t)start, (hipEvent_t)stop), "hipEventElapsedTime");
     return 0;
+}
+
+int mdxrt_copy16(void* dst, const void* src, size_t bytes, void* stream) {
+    const size_t n = bytes / 16;
+    if (bytes % 16 || ((uintptr_t)dst | (uintptr_t)src) % 16) return -1;
+    if (!n) return 0;
+    size_t blocks = (n + 255) / 256;
+    if (blocks > 512) blocks = 512;
+    k_copy16<<<dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream>>>((uint4*)dst, (const uint4*)src, n);
+    MDX_CHECK(hipGetLastError(), "k_copy16");
+    return 0;
+}
+
+int mdxrt_signal(int* flag, void* stream) {
+    k_signal<<<dim3(1), dim3(64), 0, (hipStream_t)stream>>>(flag);
+    MDX_CHECK(hipGetLastError(), "k_signal");
+    return 0;
+}
+
+// Polling sees a finished kernel about 5 us before hipStreamSynchronize
+// returns (an empty kernel 5.7 against 11.2 us).  Past 10 ms of polling the
+// stream is waited for instead, which also reports what went wrong on it.
+int mdxrt_wait(int* flag, void* stream) {
+    const auto t0 = std::chrono::steady_clock::now();
+    for (;;) {
+        for (int i = 0; i < 64; i++) {
+            if (__atomic_load_n(flag, __ATOMIC_ACQUIRE)) return 0;
+            __builtin_ia32_pause();
+        }
+        if (std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(10)) break;
+    }
+    MDX_CHECK(hipStreamSynchronize((hipStream_t)stream), "hipStreamSynchronize");
+    if (__atomic_load_n(flag, __ATOMIC_ACQUIRE)) return 0;
+    std::snprintf(g_last_error, sizeof g_last_error, "mdxrt_wait: the stream is idle but did not signal");
+    return -4;
 }
 
 int mdxrt_fill_u32(void* dst, uint32_t value, size_t n, void* stream) {
