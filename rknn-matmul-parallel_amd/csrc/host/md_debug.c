@@ -434,7 +434,7 @@ int mdx_debug_lmhead(int lm_kind, int K, int N, const void* w_rows, const float*
     d.w = dw;
     d.scale = (const float*)ds;
     d.kind = lm_kind == 1 ? MDX_W_I8 : (lm_kind == 3 ? MDX_W_F32 : MDX_W_F16);
-    if (!rc) rc = mdx_launch_lmhead(dh, dn, eps, &d, dl, dp, st, NULL, 0, s.stream);
+    if (!rc) rc = mdx_launch_lmhead(dh, dn, eps, &d, dl, dp, st, NULL, 0, NULL, s.stream);
     if (!rc) rc = mdxrt_stream_sync(s.stream);
     if (!rc) rc = mdxrt_d2h(logits, dl, (size_t)N * 4);
     mdx_state h;

@@ -33,6 +33,9 @@ typedef struct {
     void* exec;
 } md_pgraph;
 
+#define UP_SLOTS 8
+#define UP_BYTES (1 << 20)
+
 struct MatmulDecoderContext {
     MatmulDecoderConfig config;
     QuantizationType quant_type;
@@ -52,7 +55,7 @@ struct MatmulDecoderContext {
     md_layer* layers;
     uint16_t *d_kc, *d_vc;
     float *d_cos, *d_sin;
-    float *d_hidden, *d_emb_in, *d_qkv, *d_logits, *d_tmp;
+    float *d_hidden, *d_qkv, *d_logits, *d_tmp;
     void* d_sscr;                /* sampler scratch */
     void* d_part;            /* attention split partials + merge counters */
     uint16_t *d_attn16, *d_act16;
@@ -61,7 +64,7 @@ struct MatmulDecoderContext {
     int tokens_cap;
     float *d_bhidden, *d_bqkv, *d_bq, *d_gscr;
     uint16_t *d_bx16, *d_battn16, *d_bact16;
-    void *g_layers, *g_head, *g_adv, *g_greedy;
+    void *g_layers, *g_step, *g_greedy;
     int graphs_ready;
     md_pgraph pgraphs[4];
     int pgraph_next;
@@ -88,9 +91,17 @@ struct MatmulDecoderContext {
     mdx_state* h_state;
     float* h_io;
     int* h_samp;                 /* pinned: sampler tokens, then {token, kept} */
-    int* h_res;                  /* pinned: a host-fed step's {argmax, timeout flag} */
+    /* pinned, one allocation: what a step reads from and leaves for the host */
+    void* h_ctl;
+    mdx_host_res* h_res;
+    mdx_state* h_in;
+    float* h_emb;
+    float clock_ms;              /* ms per tick of the times in h_res */
     size_t h_io_floats;
-    void *ev0, *ev1, *ev2;
+    float* h_up;                 /* pinned ring of UP_SLOTS pieces: a long prompt on its way up */
+    size_t up_floats;            /* per piece */
+    void* up_ev[UP_SLOTS];       /* the piece's copy is done */
+    void *ev0, *ev1;
     MatmulDecoderStats stats;
 };
 
@@ -369,7 +380,6 @@ static int layout(MatmulDecoderContext* c, const md_source* s) {
     const int nlog = c->V > c->lm_vocab ? c->V : c->lm_vocab;
     const int widest = c->qd + 2 * c->kvd > 2 * c->F ? c->qd + 2 * c->kvd : 2 * c->F;
     CARVE(c->d_hidden, (size_t)c->d * 4);
-    CARVE(c->d_emb_in, (size_t)c->d * 4);
     CARVE(c->d_qkv, (size_t)(c->qd + 2 * c->kvd) * 4);
     CARVE(c->d_part, mdx_attn_decode_scratch_bytes(c->nq, c->nkv, c->hd, c->max_splits));
     CARVE(c->d_logits, (size_t)nlog * 4);
@@ -521,13 +531,16 @@ static int upload_lm_single(MatmulDecoderContext* c, const float* lm32) {
 /* Launch sequences                                                          */
 /* ------------------------------------------------------------------------ */
 
-static int run_layers(MatmulDecoderContext* c, void* s) {
+/* fed: the step's state and embedding come from pinned memory (h_in, h_emb),
+ * else from the device state. */
+static int run_layers(MatmulDecoderContext* c, int fed, void* s) {
     const float eps = c->config.rms_eps;
     int rc = 0;
     for (int l = 0; l < c->L && rc == 0; l++) {
         md_layer* ly = &c->layers[l];
         if (l == 0)
-            rc = mdx_launch_embed_norm_gemv(c->d_state, c->d_emb, c->d_emb_in, c->V, c->d_hidden,
+            rc = mdx_launch_embed_norm_gemv(fed ? c->h_in : c->d_state, fed ? c->d_state : NULL,
+                                            fed ? c->h_res : NULL, c->d_emb, c->h_emb, c->V, c->d_hidden,
                                             ly->in_norm, eps, &ly->qkv, c->d_qkv, s);
         else
             rc = mdx_launch_norm_gemv(c->d_hidden, ly->in_norm, eps, &ly->qkv, 0, c->d_qkv, s);
@@ -543,10 +556,10 @@ static int run_layers(MatmulDecoderContext* c, void* s) {
     return rc;
 }
 
-static int run_head(MatmulDecoderContext* c, const mdx_wdesc* lm, int* out_tokens, int advance,
-                    void* s) {
-    return mdx_launch_lmhead(c->d_hidden, c->d_final_norm, c->config.rms_eps, lm, c->d_logits,
-                             c->d_partial, c->d_state, out_tokens, advance, s);
+static int run_head(MatmulDecoderContext* c, const mdx_wdesc* lm, float* logits, int* out_tokens,
+                    int advance, mdx_host_res* res, void* s) {
+    return mdx_launch_lmhead(c->d_hidden, c->d_final_norm, c->config.rms_eps, lm, logits,
+                             c->d_partial, c->d_state, out_tokens, advance, res, s);
 }
 
 static int run_prefill(MatmulDecoderContext* c, int M, void* s) {
@@ -619,12 +632,17 @@ static int capture(MatmulDecoderContext* c, md_seq_fn fn, void** exec) {
     return rc2 ? rc2 : rc;
 }
 
-static int seq_layers(MatmulDecoderContext* c, void* s) { return run_layers(c, s); }
-static int seq_head(MatmulDecoderContext* c, void* s) { return run_head(c, &c->lm, NULL, 1, s); }
-static int seq_adv(MatmulDecoderContext* c, void* s) { return mdx_launch_advance(c->d_state, 1, s); }
+static int seq_layers(MatmulDecoderContext* c, void* s) { return run_layers(c, 1, s); }
+/* a whole host-fed step: logits, argmax and the done word to pinned memory */
+static int seq_step(MatmulDecoderContext* c, void* s) {
+    int rc = run_layers(c, 1, s);
+    if (!rc) rc = run_head(c, &c->lm, c->h_io, NULL, 1, c->h_res, s);
+    if (!rc) rc = mdxrt_signal(&c->h_res->done, &c->h_res->t_end, s);
+    return rc;
+}
 static int seq_greedy(MatmulDecoderContext* c, void* s) {
-    int rc = run_layers(c, s);
-    if (!rc) rc = run_head(c, &c->lm, c->d_tokens, 1, s);
+    int rc = run_layers(c, 0, s);
+    if (!rc) rc = run_head(c, &c->lm, c->d_logits, c->d_tokens, 1, NULL, s);
     return rc;
 }
 
@@ -640,9 +658,9 @@ static int ensure_graphs(MatmulDecoderContext* c) {
         c->graphs_ready = 1;
         return 0;
     }
-    int rc = capture(c, seq_layers, &c->g_layers);
-    if (!rc && c->n_lm <= 1) rc = capture(c, seq_head, &c->g_head);
-    if (!rc) rc = capture(c, seq_adv, &c->g_adv);
+    /* a one-launch step replays nothing */
+    int rc = c->persist ? 0 : capture(c, seq_layers, &c->g_layers);
+    if (!rc && !c->persist && c->n_lm <= 1) rc = capture(c, seq_step, &c->g_step);
     if (rc) {
         fprintf(stderr, "[MatmulDecoder] graph capture failed: %s\n", mdxrt_last_error());
         return MATMUL_DECODER_ERR_RKNN;
@@ -739,7 +757,7 @@ static void setup_persist(MatmulDecoderContext* c) {
     a->layer_stride = stride;
     a->kv_stride = (long long)c->max_seq * c->kvd;
     a->emb_table = c->d_emb;
-    a->emb_in = c->d_emb_in;
+    a->emb_in = c->h_emb;
     a->cos_t = c->d_cos;
     a->sin_t = c->d_sin;
     a->final_norm = c->d_final_norm;
@@ -900,7 +918,7 @@ static MatmulDecoderContext* create_common(const MatmulDecoderConfig* config,
     if (!c->layers || (c->n_lm && !c->lm_heads)) goto fail;
 
     if (mdxrt_stream_create(&c->stream) || mdxrt_event_create(&c->ev0) ||
-        mdxrt_event_create(&c->ev1) || mdxrt_event_create(&c->ev2))
+        mdxrt_event_create(&c->ev1))
         goto fail;
 
     /* size, allocate, then lay out for real */
@@ -966,8 +984,21 @@ static MatmulDecoderContext* create_common(const MatmulDecoderConfig* config,
     c->h_io_floats = (size_t)(c->V > c->lm_vocab ? c->V : c->lm_vocab);
     if ((size_t)c->max_m * c->d > c->h_io_floats) c->h_io_floats = (size_t)c->max_m * c->d;
     if (mdxrt_host_alloc((void**)&c->h_io, c->h_io_floats * 4)) goto fail;
+    if (c->long_m) {
+        const size_t all = (size_t)c->long_m * c->d;
+        c->up_floats = UP_BYTES / 4;
+        if (c->up_floats > (all + UP_SLOTS - 1) / UP_SLOTS) c->up_floats = (all + UP_SLOTS - 1) / UP_SLOTS;
+        if (mdxrt_host_alloc((void**)&c->h_up, c->up_floats * UP_SLOTS * 4)) goto fail;
+        for (int i = 0; i < UP_SLOTS; i++)
+            if (mdxrt_event_create(&c->up_ev[i])) goto fail;
+    }
     if (mdxrt_host_alloc((void**)&c->h_samp, (MDX_SAMPLE_MAX_REPEAT + 64) * sizeof(int))) goto fail;
-    if (mdxrt_host_alloc((void**)&c->h_res, 4 * sizeof(int))) goto fail;
+    if (mdxrt_host_alloc(&c->h_ctl, 512 + (size_t)c->d * 4)) goto fail;
+    memset(c->h_ctl, 0, 512 + (size_t)c->d * 4);
+    c->h_res = (mdx_host_res*)c->h_ctl;
+    c->h_in = (mdx_state*)((char*)c->h_ctl + 256);
+    c->h_emb = (float*)((char*)c->h_ctl + 512);
+    c->clock_ms = 1.0f / (float)mdxrt_clock_khz();
     memset(c->h_state, 0, sizeof(mdx_state));
     setup_persist(c);
     {
@@ -1054,8 +1085,7 @@ void matmul_decoder_destroy(MatmulDecoderContext* c) {
     if (!c) return;
     if (c->stream) mdxrt_stream_sync(c->stream);
     mdxrt_graph_destroy(c->g_layers);
-    mdxrt_graph_destroy(c->g_head);
-    mdxrt_graph_destroy(c->g_adv);
+    mdxrt_graph_destroy(c->g_step);
     mdxrt_graph_destroy(c->g_greedy);
     for (int i = 0; i < 4; i++) mdxrt_graph_destroy(c->pgraphs[i].exec);
     mdxrt_free(c->d_tokens);
@@ -1066,10 +1096,11 @@ void matmul_decoder_destroy(MatmulDecoderContext* c) {
     mdxrt_host_free(c->h_state);
     mdxrt_host_free(c->h_io);
     mdxrt_host_free(c->h_samp);
-    mdxrt_host_free(c->h_res);
+    mdxrt_host_free(c->h_up);
+    for (int i = 0; i < UP_SLOTS; i++) mdxrt_event_destroy(c->up_ev[i]);
+    mdxrt_host_free(c->h_ctl);
     mdxrt_event_destroy(c->ev0);
     mdxrt_event_destroy(c->ev1);
-    mdxrt_event_destroy(c->ev2);
     mdxrt_stream_destroy(c->stream);
     free(c->layers);
     free(c->lm_heads);
@@ -1080,18 +1111,15 @@ void matmul_decoder_destroy(MatmulDecoderContext* c) {
 /* Steps                                                                     */
 /* ------------------------------------------------------------------------ */
 
-static int set_state(MatmulDecoderContext* c, int token_id, const float* embedding) {
-    memset(c->h_state, 0, sizeof(mdx_state));
-    c->h_state->pos = c->seq_len;
-    c->h_state->token = embedding ? 0 : token_id;
-    c->h_state->mode = embedding ? 1 : 0;
-    int rc = 0;
-    if (embedding) {
-        memcpy(c->h_io, embedding, (size_t)c->d * 4);
-        rc = mdxrt_h2d_async(c->d_emb_in, c->h_io, (size_t)c->d * 4, c->stream);
-    }
-    if (!rc) rc = mdxrt_h2d_async(c->d_state, c->h_state, sizeof(mdx_state), c->stream);
-    return rc;
+/* The input of the next step, in pinned memory. */
+static void feed(MatmulDecoderContext* c, int token_id, const float* embedding) {
+    memset(c->h_res, 0, sizeof *c->h_res);
+    c->h_res->argmax = -1;
+    memset(c->h_in, 0, sizeof(mdx_state));
+    c->h_in->pos = c->seq_len;
+    c->h_in->token = embedding ? 0 : token_id;
+    c->h_in->mode = embedding ? 1 : 0;
+    if (embedding) memcpy(c->h_emb, embedding, (size_t)c->d * 4);
 }
 
 /* Shared by step and step_head: validation order of the reference
@@ -1106,9 +1134,6 @@ static int step_checks(MatmulDecoderContext* c, int token_id, const float* embed
     return 0;
 }
 
-/* One decode step.  want_head selects the lm_head (the reference's
- * output_logits != NULL); logits_out may be NULL with want_head set when
- * only the token is needed. */
 /* A device-side draw appended to a step (matmul_decoder_step_sample): the n
  * distinct penalised tokens are in c->h_samp[0..n). */
 typedef struct {
@@ -1183,65 +1208,46 @@ static int trace_arm(MatmulDecoderContext* c) {
     return mdxrt_fill_u32(c->d_trace, 0u, (size_t)256 * c->trace_ev * 2, c->stream);
 }
 
-static int do_step(MatmulDecoderContext* c, int token_id, const float* embedding,
-                   float* output_logits, int want_head, const md_sample_req* sr) {
-    if (!c) return MATMUL_DECODER_ERR_INVALID_ARG;
+/* One decode step with the lm_head `lm` (NULL: none, the reference's
+ * output_logits == NULL); output_logits may be NULL when only the token is
+ * needed.  Nothing is copied before or after the kernels: the first one reads
+ * the position, token and embedding in pinned memory (the one launch takes all
+ * but the embedding as arguments), the last ones store the logits, the argmax
+ * and the times there, and the host polls the done word.  A sampling step
+ * keeps its logits on the device for the sampler. */
+static int run_step(MatmulDecoderContext* c, int token_id, const float* embedding, const mdx_wdesc* lm,
+                    float* output_logits, const md_sample_req* sr, int count) {
     const double t0 = md_now_ms();
     int rc = step_checks(c, token_id, embedding);
     if (rc) return rc;
     if (ensure_graphs(c)) return MATMUL_DECODER_ERR_RKNN;
-    if (c->n_lm > 1 && want_head) {
-        /* multi-head model: the reference step() has no single lm_head
-         * either; use head 0 like step_head(…, 0, …) */
-        return matmul_decoder_step_head(c, token_id, embedding, 0, output_logits);
-    }
-    const int prof = c->profile && c->persist && c->d_trace;
-    const int one_launch_head = c->persist && c->persist_head && want_head;
-    /* A step with the head in the one launch is host-fed: the position, token
-     * and mode go in as kernel arguments, and the kernel writes the argmax,
-     * the timeout flag and (for a plain step) the logits to mapped host
-     * memory, so no copy runs before or after it.  A sampling step keeps its
-     * logits on the device for the sampler (and copies them out when asked);
-     * a profiling step keeps every copy. */
-    const int host_fed = one_launch_head && !prof && (long long)c->V <= 256LL * 1024;
-    const int host_logits = host_fed && !sr && output_logits;
+    const int prof = count && c->profile && c->persist && c->d_trace;
+    const int one = c->persist && c->persist_head && lm == &c->lm;   /* the head in the one launch */
+    const int V = lm == &c->lm ? c->V : c->lm_vocab;
+    /* the one launch stages a workgroup's logits in LDS on their way to the host */
+    const int host_logits = output_logits && !sr && (!one || (long long)V <= 256LL * 1024);
+    float* const logits = host_logits ? c->h_io : c->d_logits;
     if (c->persist) pthread_mutex_lock(&g_persist_mu);
-    if (host_fed) {
-        c->h_res[0] = -1;
-        c->h_res[1] = 0;
+    feed(c, token_id, embedding);
+    rc = prof ? trace_arm(c) : 0;
+    if (c->persist) {
         c->pargs.in_args = 1;
-        c->pargs.in_pos = c->seq_len;
-        c->pargs.in_token = embedding ? 0 : token_id;
-        c->pargs.in_mode = embedding ? 1 : 0;
+        c->pargs.in_pos = c->h_in->pos;
+        c->pargs.in_token = c->h_in->token;
+        c->pargs.in_mode = c->h_in->mode;
         c->pargs.res_host = c->h_res;
-        c->pargs.logits_host = host_logits ? c->h_io : NULL;
-        rc = 0;
-        if (embedding) {
-            memcpy(c->h_io, embedding, (size_t)c->d * 4);
-            rc = mdxrt_h2d_async(c->d_emb_in, c->h_io, (size_t)c->d * 4, c->stream);
-        }
+        c->pargs.logits_host = one && host_logits ? c->h_io : NULL;
+        if (!rc) rc = launch_persist(c, one, NULL, c->seq_len);
+        /* a head of its own: the launch above has advanced the position */
+        if (!rc && lm && !one) rc = run_head(c, lm, logits, NULL, 0, c->h_res, c->stream);
+    } else if (lm == &c->lm && !sr) {
+        rc = launch_seq(c, c->g_step, seq_step);
     } else {
-        rc = set_state(c, token_id, embedding);
+        rc = launch_seq(c, c->g_layers, seq_layers);
+        if (!rc && lm) rc = run_head(c, lm, logits, NULL, 1, c->h_res, c->stream);
     }
-    if (!rc && prof) rc = trace_arm(c);
-    if (!rc) rc = mdxrt_event_record(c->ev0, c->stream);
-    if (c->persist && (c->persist_head || !want_head)) {
-        if (!rc) rc = launch_persist(c, want_head, NULL, c->seq_len);
-        if (!rc) rc = mdxrt_event_record(c->ev1, c->stream);
-    } else if (c->persist) {
-        /* the fp16 lm_head: layers in one launch (which advances the
-         * position), then the per-stage head */
-        if (!rc) rc = launch_persist(c, 0, NULL, c->seq_len);
-        if (!rc) rc = mdxrt_event_record(c->ev1, c->stream);
-        if (!rc) rc = run_head(c, &c->lm, NULL, 0, c->stream);
-    } else {
-        if (!rc) rc = launch_seq(c, c->g_layers, seq_layers);
-        if (!rc) rc = mdxrt_event_record(c->ev1, c->stream);
-        if (!rc) rc = launch_seq(c, want_head ? c->g_head : c->g_adv, want_head ? seq_head : seq_adv);
-    }
-    if (!rc) rc = mdxrt_event_record(c->ev2, c->stream);
     if (!rc && output_logits && !host_logits)
-        rc = mdxrt_d2h_async(c->h_io, c->d_logits, (size_t)c->V * 4, c->stream);
+        rc = mdxrt_d2h_async(c->h_io, c->d_logits, (size_t)V * 4, c->stream);
     if (!rc && sr) {
         /* penalty and draw on the logits just copied out; the kernels read
          * the tokens from and write {token, kept} to pinned host memory */
@@ -1252,56 +1258,61 @@ static int do_step(MatmulDecoderContext* c, int token_id, const float* embedding
                                         c->d_sscr, c->h_samp + MDX_SAMPLE_MAX_REPEAT, NULL, NULL,
                                         c->stream);
     }
-    if (!rc && !host_fed) rc = mdxrt_d2h_async(c->h_state, c->d_state, sizeof(mdx_state), c->stream);
     if (!rc && prof)
         rc = mdxrt_d2h_async(c->h_trace, c->d_trace, (size_t)256 * c->trace_ev * 8, c->stream);
-    if (!rc) rc = mdxrt_stream_sync(c->stream);
+    if (!rc && !(!c->persist && lm == &c->lm && !sr)) rc = mdxrt_signal(&c->h_res->done, &c->h_res->t_end, c->stream);
+    if (!rc) rc = mdxrt_wait(&c->h_res->done, c->stream);
+    if (rc) mdxrt_stream_sync(c->stream);
     c->pargs.trace = NULL;
     c->pargs.trace_stride = 0;
     c->pargs.in_args = 0;
     c->pargs.res_host = NULL;
     c->pargs.logits_host = NULL;
-    if (host_fed && !rc) {
-        c->h_state->pad[1] = c->h_res[1];
-        c->h_state->argmax = c->h_res[0];
-    }
     if (c->persist) pthread_mutex_unlock(&g_persist_mu);
     if (rc) {
         fprintf(stderr, "[MatmulDecoder] step failed: %s\n", mdxrt_last_error());
         return MATMUL_DECODER_ERR_RKNN;
     }
-    if (c->h_state->pad[1]) {
-        if (persist_retry(c)) return do_step(c, token_id, embedding, output_logits, want_head, sr);
+    if (c->h_res->timeout) {
+        if (persist_retry(c)) return run_step(c, token_id, embedding, lm, output_logits, sr, count);
         fprintf(stderr, "[MatmulDecoder] step failed: a workgroup timed out waiting for another\n");
         return MATMUL_DECODER_ERR_RKNN;
     }
-    float layers_ms = 0.0f, head_ms = 0.0f;
-    mdxrt_event_elapsed_ms(c->ev0, c->ev1, &layers_ms);
-    mdxrt_event_elapsed_ms(c->ev1, c->ev2, &head_ms);
     c->seq_len++;
-    int tok = 0;
-    if (output_logits) memcpy(output_logits, c->h_io, (size_t)c->V * 4);
-    if (want_head) tok = c->h_state->argmax;
-    if (sr) tok = c->h_samp[MDX_SAMPLE_MAX_REPEAT];
+    if (output_logits) memcpy(output_logits, c->h_io, (size_t)V * 4);
+    const int tok = sr ? c->h_samp[MDX_SAMPLE_MAX_REPEAT] : (lm ? c->h_res->argmax : 0);
+    if (!count) return tok;
     const float total = (float)(md_now_ms() - t0);
-    /* Device times from events on the step's stream: layers_ms is the layers
-     * launch (with the lm_head too when it runs inside it), head_ms the
-     * separate head kernels.  Without MDX_PROFILE the one launch is not split:
-     * it all counts as matmul_ms. */
+    /* Device times from the kernels: layers_ms is the layers' (with the lm_head
+     * too when it runs inside the one launch), head_ms the rest.  Without
+     * MDX_PROFILE the one launch is not split: it all counts as matmul_ms. */
+    const mdx_host_res* r = c->h_res;
+    const unsigned long long mid = r->t_layers ? r->t_layers : r->t_end;
+    const float layers_ms = (float)(mid - r->t_start) * c->clock_ms;
+    const float head_ms = (float)(r->t_end - mid) * c->clock_ms;
     c->stats.total_ms = total;
     c->stats.matmul_ms = layers_ms;
     c->stats.rebind_ms = 0.0f;
     c->stats.cpu_ops_ms = 0.0f;
-    c->stats.lm_head_ms = want_head && !one_launch_head ? head_ms : 0.0f;
+    c->stats.lm_head_ms = lm && !one ? head_ms : 0.0f;
     if (prof) {
-        profile_split(c, layers_ms, one_launch_head, &c->stats);
-        if (want_head && !one_launch_head) c->stats.lm_head_ms = head_ms;
+        profile_split(c, layers_ms, one, &c->stats);
+        if (lm && !one) c->stats.lm_head_ms = head_ms;
     }
     c->stats.convert_ms = total - c->stats.matmul_ms - c->stats.cpu_ops_ms - c->stats.rebind_ms -
                           c->stats.lm_head_ms;
     if (c->stats.convert_ms < 0) c->stats.convert_ms = 0;
     c->stats.n_steps++;
     return tok;
+}
+
+static int do_step(MatmulDecoderContext* c, int token_id, const float* embedding,
+                   float* output_logits, int want_head, const md_sample_req* sr) {
+    if (!c) return MATMUL_DECODER_ERR_INVALID_ARG;
+    /* multi-head model: the reference step() has no single lm_head either; head
+     * 0 like step_head(..., 0, ...) */
+    if (c->n_lm > 1 && want_head) return run_step(c, token_id, embedding, &c->lm_heads[0], output_logits, NULL, 0);
+    return run_step(c, token_id, embedding, want_head ? &c->lm : NULL, output_logits, sr, 1);
 }
 
 int matmul_decoder_step(MatmulDecoderContext* c, int token_id, const float* embedding,
@@ -1324,56 +1335,55 @@ int matmul_decoder_step_head(MatmulDecoderContext* c, int token_id, const float*
     if (!c) return MATMUL_DECODER_ERR_INVALID_ARG;
     if (c->n_lm <= 1) return matmul_decoder_step(c, token_id, embedding, output_logits);
     if (lm_head_idx < 0 || lm_head_idx >= c->n_lm) return MATMUL_DECODER_ERR_INVALID_ARG;
-    int rc = step_checks(c, token_id, embedding);
-    if (rc) return rc;
-    if (ensure_graphs(c)) return MATMUL_DECODER_ERR_RKNN;
-    if (c->persist) pthread_mutex_lock(&g_persist_mu);
-    rc = set_state(c, token_id, embedding);
-    if (c->persist) {
-        /* the one launch advances the position; the head does not */
-        if (!rc) rc = launch_persist(c, 0, NULL, c->seq_len);
-        if (!rc) rc = run_head(c, &c->lm_heads[lm_head_idx], NULL, 0, c->stream);
-    } else {
-        if (!rc) rc = launch_seq(c, c->g_layers, seq_layers);
-        if (!rc) rc = run_head(c, &c->lm_heads[lm_head_idx], NULL, 1, c->stream);
-    }
-    if (!rc && output_logits)
-        rc = mdxrt_d2h_async(c->h_io, c->d_logits, (size_t)c->lm_vocab * 4, c->stream);
-    if (!rc) rc = mdxrt_d2h_async(c->h_state, c->d_state, sizeof(mdx_state), c->stream);
-    if (!rc) rc = mdxrt_stream_sync(c->stream);
-    if (c->persist) pthread_mutex_unlock(&g_persist_mu);
-    if (rc) return MATMUL_DECODER_ERR_RKNN;
-    if (c->h_state->pad[1]) {
-        if (persist_retry(c)) return matmul_decoder_step_head(c, token_id, embedding, lm_head_idx, output_logits);
-        fprintf(stderr, "[MatmulDecoder] step failed: a workgroup timed out waiting for another\n");
-        return MATMUL_DECODER_ERR_RKNN;
-    }
-    c->seq_len++;
-    if (output_logits) memcpy(output_logits, c->h_io, (size_t)c->lm_vocab * 4);
-    return c->h_state->argmax;
+    return run_step(c, token_id, embedding, &c->lm_heads[lm_head_idx], output_logits, NULL, 0);
 }
 
+/* Up to max_m rows; returns with the stream idle. */
 static int prefill_chunk(MatmulDecoderContext* c, const float* emb, int M) {
+    memcpy(c->h_io, emb, (size_t)M * c->d * 4);
     memset(c->h_state, 0, sizeof(mdx_state));
     c->h_state->pos = c->seq_len;
+    c->h_res->done = 0;
+    int rc = mdxrt_h2d_async(c->d_bhidden, c->h_io, (size_t)M * c->d * 4, c->stream);
+    if (!rc) rc = mdxrt_h2d_async(c->d_state, c->h_state, sizeof(mdx_state), c->stream);
+    void* g = rc ? NULL : prefill_graph(c, M);
+    if (!rc) rc = g ? mdxrt_graph_launch(g, c->stream) : run_prefill(c, M, c->stream);
+    if (!rc) rc = mdxrt_signal(&c->h_res->done, NULL, c->stream);
+    if (!rc) rc = mdxrt_wait(&c->h_res->done, c->stream);
+    return rc;
+}
+
+/* Any number of rows, in equal passes of up to long_m (one of a few rows would
+ * read all weights for them).  A pass's rows go up in pieces of about 1 MB:
+ * the host fills one while others are copied, and the next pass's first ones
+ * while this pass runs (4000 rows of 1024: 16 MB, 480 us through the runtime's
+ * pageable copy). */
+static int prefill_long(MatmulDecoderContext* c, const float* emb, int M) {
+    const int n = (M + c->long_m - 1) / c->long_m, step = (M + n - 1) / n;
+    memset(c->h_state, 0, sizeof(mdx_state));
+    c->h_state->pos = c->seq_len;
+    c->h_res->done = 0;
     int rc = mdxrt_h2d_async(c->d_state, c->h_state, sizeof(mdx_state), c->stream);
-    if (M <= c->max_m) {
-        memcpy(c->h_io, emb, (size_t)M * c->d * 4);
-        if (!rc) rc = mdxrt_h2d_async(c->d_bhidden, c->h_io, (size_t)M * c->d * 4, c->stream);
-        void* g = rc ? NULL : prefill_graph(c, M);
-        if (!rc) rc = g ? mdxrt_graph_launch(g, c->stream) : run_prefill(c, M, c->stream);
-    } else {
-        if (!rc) rc = mdxrt_h2d_async(c->d_bhidden, emb, (size_t)M * c->d * 4, c->stream);
-        if (!rc) rc = run_prefill_long(c, M, c->seq_len, c->stream);
+    unsigned piece = 0;
+    for (int off = 0; off < M && !rc; off += step) {
+        const int m = M - off < step ? M - off : step;
+        const float* src = emb + (size_t)off * c->d;
+        const size_t total = (size_t)m * c->d;
+        for (size_t at = 0; at < total && !rc; at += c->up_floats, piece++) {
+            const size_t k = total - at < c->up_floats ? total - at : c->up_floats;
+            const unsigned slot = piece % UP_SLOTS;
+            float* h = c->h_up + (size_t)slot * c->up_floats;
+            if (piece >= UP_SLOTS) rc = mdxrt_event_sync(c->up_ev[slot]);
+            memcpy(h, src + at, k * 4);
+            if (!rc) rc = mdxrt_h2d_async(c->d_bhidden + at, h, k * 4, c->stream);
+            if (!rc) rc = mdxrt_event_record(c->up_ev[slot], c->stream);
+        }
+        if (!rc) rc = run_prefill_long(c, m, c->seq_len + off, c->stream);
+        c->last_row = m - 1;
     }
-    if (!rc) rc = mdxrt_stream_sync(c->stream);
-    if (rc) {
-        fprintf(stderr, "[BatchPrefill] failed: %s\n", mdxrt_last_error());
-        return MATMUL_DECODER_ERR_RKNN;
-    }
-    c->seq_len += M;
-    c->last_row = M - 1;
-    return 0;
+    if (!rc) rc = mdxrt_signal(&c->h_res->done, NULL, c->stream);
+    if (!rc) rc = mdxrt_wait(&c->h_res->done, c->stream);
+    return rc;
 }
 
 int matmul_decoder_prefill_batch(MatmulDecoderContext* c, const float* embeddings, int M) {
@@ -1383,16 +1393,19 @@ int matmul_decoder_prefill_batch(MatmulDecoderContext* c, const float* embedding
                 M, c->max_seq);
         return MATMUL_DECODER_ERR_INVALID_ARG;
     }
-    /* equal passes (one of a few rows would read all weights for them) */
-    int step = c->max_m;
-    if (M > c->max_m && c->long_m) {
-        const int n = (M + c->long_m - 1) / c->long_m;
-        step = (M + n - 1) / n;
-    }
+    const int lng = M > c->max_m && c->long_m;
+    const int step = lng ? M : c->max_m;
     for (int off = 0; off < M; off += step) {
         const int n = M - off < step ? M - off : step;
-        int rc = prefill_chunk(c, embeddings + (size_t)off * c->d, n);
-        if (rc) return rc;
+        const float* e = embeddings + (size_t)off * c->d;
+        const int rc = lng ? prefill_long(c, e, n) : prefill_chunk(c, e, n);
+        if (rc) {
+            mdxrt_stream_sync(c->stream);
+            fprintf(stderr, "[BatchPrefill] failed: %s\n", mdxrt_last_error());
+            return MATMUL_DECODER_ERR_RKNN;
+        }
+        c->seq_len += n;
+        if (!lng) c->last_row = n - 1;
     }
     return MATMUL_DECODER_OK;
 }
@@ -1548,13 +1561,13 @@ int mdx_prefill_logits(MatmulDecoderContext* c, const float* embeddings, int M, 
     int rc = matmul_decoder_prefill_batch(c, embeddings, M);
     if (rc) return rc;
     rc = mdx_launch_copy_row(c->d_bhidden, c->last_row, c->d, c->d_hidden, c->stream);
-    if (!rc) rc = run_head(c, &c->lm, NULL, 0, c->stream);
-    if (!rc && logits) rc = mdxrt_d2h_async(c->h_io, c->d_logits, (size_t)c->V * 4, c->stream);
-    if (!rc) rc = mdxrt_d2h_async(c->h_state, c->d_state, sizeof(mdx_state), c->stream);
-    if (!rc) rc = mdxrt_stream_sync(c->stream);
+    memset(c->h_res, 0, sizeof *c->h_res);
+    if (!rc) rc = run_head(c, &c->lm, c->h_io, NULL, 0, c->h_res, c->stream);
+    if (!rc) rc = mdxrt_signal(&c->h_res->done, NULL, c->stream);
+    if (!rc) rc = mdxrt_wait(&c->h_res->done, c->stream);
     if (rc) return MATMUL_DECODER_ERR_RKNN;
     if (logits) memcpy(logits, c->h_io, (size_t)c->V * 4);
-    return c->h_state->argmax;
+    return c->h_res->argmax;
 }
 
 int mdx_generate_greedy(MatmulDecoderContext* c, int first_token, int n_steps, int* out_tokens,
@@ -1588,7 +1601,7 @@ int mdx_generate_greedy(MatmulDecoderContext* c, int first_token, int n_steps, i
             rc = launch_persist(c, 1, c->d_tokens, c->seq_len + i);
         } else {
             rc = launch_persist(c, 0, NULL, c->seq_len + i);
-            if (!rc) rc = run_head(c, &c->lm, c->d_tokens, 0, c->stream);
+            if (!rc) rc = run_head(c, &c->lm, c->d_logits, c->d_tokens, 0, NULL, c->stream);
         }
     }
     if (!rc) rc = mdxrt_event_record(c->ev1, c->stream);
@@ -1670,7 +1683,7 @@ static int time_projection_launch(MatmulDecoderContext* c, int sel, int l, const
             break;
         default:
             rc = mdx_launch_lmhead(c->d_hidden, c->d_final_norm, eps, w0, c->d_logits,
-                                   c->d_partial, c->d_state, NULL, 0, c->stream);
+                                   c->d_partial, c->d_state, NULL, 0, NULL, c->stream);
     }
     return rc;
 }
@@ -1754,7 +1767,10 @@ int mdx_trace_step(MatmulDecoderContext* c, int token_id, unsigned long long* ou
     unsigned long long* d = NULL;
     if (mdxrt_malloc((void**)&d, (size_t)256 * ev * 8)) return MATMUL_DECODER_ERR_MEMORY;
     pthread_mutex_lock(&g_persist_mu);
-    rc = set_state(c, token_id, NULL);
+    memset(c->h_state, 0, sizeof(mdx_state));
+    c->h_state->pos = c->seq_len;
+    c->h_state->token = token_id;
+    rc = mdxrt_h2d_async(c->d_state, c->h_state, sizeof(mdx_state), c->stream);
     if (!rc) rc = mdxrt_fill_u32(d, 0u, (size_t)256 * ev * 2, c->stream);
     c->pargs.trace = d;
     c->pargs.trace_stride = ev;

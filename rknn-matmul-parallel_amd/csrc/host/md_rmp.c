@@ -149,7 +149,7 @@ static int rmp_issue(RmpContext* c, const int16_t* input, int p) {
     if (c->config.M == 1) rc = mdx_launch_gemv_f16in(x, &c->w, hy, s);
     else for (int r0 = 0; r0 < mm && !rc; r0 += 64)
         rc = mdx_launch_gemm(x + (size_t)r0 * Kp, mm - r0 < 64 ? mm - r0 : 64, &c->w, 0, hy + (size_t)r0 * N, NULL, s);
-    return rc ? rc : mdxrt_signal(&c->h_flag[slot], s);
+    return rc ? rc : mdxrt_signal(&c->h_flag[slot], NULL, s);
 }
 
 /* memcpy; a large block, which the GPU has just written past the caches, with

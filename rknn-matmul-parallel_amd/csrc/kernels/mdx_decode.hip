@@ -50,6 +50,8 @@ struct GemvArgs {
     uint16_t* out_f16;
     // XM_EMBED: input row chosen by state->mode / state->token, copied to hidden_out
     const mdx_state* st_in;
+    mdx_state* st_copy;      // st_in is in host memory: copied here for the kernels that follow
+    mdx_host_res* res;       // times and argmax for the host, or NULL
     const float* emb_table;
     int vocab;
     float* hidden_out;
@@ -342,8 +344,8 @@ __device__ __forceinline__ unsigned long long wave_max_key(unsigned long long be
 // The end of an lm_head launch: the workgroup's argmax key from its waves'
 // (best: wave-uniform), and, in the last workgroup to arrive, the argmax of
 // all keys and the step's bookkeeping.
-__device__ __forceinline__ void lm_finish(const GemvArgs& a, unsigned long long best, unsigned long long* bkey,
-                                          int* last_block) {
+__device__ __forceinline__ void lm_finish(const GemvArgs& a, unsigned long long t_begin, unsigned long long best,
+                                          unsigned long long* bkey, int* last_block) {
     LmScratch* scr = reinterpret_cast<LmScratch*>(a.lm_scr);
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     if (lane == 0) bkey[wave] = best;
@@ -389,7 +391,18 @@ __device__ __forceinline__ void lm_finish(const GemvArgs& a, unsigned long long 
             st->n_out = st->n_out + 1;
         }
         st->pos = st->pos + a.advance;
+        if (a.res) {
+            a.res->argmax = tok;
+            a.res->t_layers = t_begin;
+        }
     }
+}
+
+// The step's first kernel: the host's state to the device, and the time.
+__device__ __forceinline__ void step_begin(const GemvArgs& a) {
+    if (blockIdx.x != 0 || threadIdx.x != 0) return;
+    if (a.st_copy) *a.st_copy = *a.st_in;
+    if (a.res) a.res->t_start = wall_clock64();
 }
 
 // The GEMV.  Blocks of 256 threads (4 waves x RW rows) walk the row blocks
@@ -409,6 +422,7 @@ __global__ __launch_bounds__(256) void k_gemv(GemvArgs a) {
     const size_t row_bytes = (size_t)a.K * T::EB2 / 2;
     const long slots = (long)a.n_units * a.unit_rows;
     const int nblk = (int)((slots + 4L * RW - 1) / (4L * RW));
+    const unsigned long long t_begin = a.res ? wall_clock64() : 0;
     const bool single = nchunks <= 64 * U;
 
     int blk = blockIdx.x;
@@ -461,7 +475,8 @@ __global__ __launch_bounds__(256) void k_gemv(GemvArgs a) {
         if (!single && nb < nblk) rs.load(a, row_bytes, nchunks, 0, lane, wv);
     }
 
-    if (a.epi == EP_LOGITS) lm_finish(a, best, bkey, &last_block);
+    if (a.epi == EP_LOGITS) lm_finish(a, t_begin, best, bkey, &last_block);
+    else if (a.xmode == XM_EMBED) step_begin(a);
 }
 
 // The GEMV when every workgroup takes exactly one row block and a lane's
@@ -502,6 +517,7 @@ __global__ __launch_bounds__(256) void k_gemv_once(GemvArgs a) {
         if (a.scale && rs.valid[r]) y[r] = y[r] * rs.sc[r];
     }
     store_rows<KIND, RW, U>(a, rs, y, lane);
+    if (a.xmode == XM_EMBED) step_begin(a);
 }
 
 // INT8 lm_head with K = 1024 (one 16-byte chunk per lane is a whole row):
@@ -518,6 +534,7 @@ __global__ __launch_bounds__(256) void k_lmhead_i8_1k(GemvArgs a) {
     __shared__ unsigned long long bkey[4];
     __shared__ int last_block;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const unsigned long long t_begin = a.res ? wall_clock64() : 0;
     const int rb = (int)(((long long)blockIdx.x * a.N) / gridDim.x);
     const int re = (int)(((long long)(blockIdx.x + 1) * a.N) / gridDim.x);
     auto load = [&](uint4 (&w)[U], float& sc, int base) {
@@ -560,7 +577,7 @@ __global__ __launch_bounds__(256) void k_lmhead_i8_1k(GemvArgs a) {
         if (base + 16 * U < re) load(w1, sc1, base + 16 * U);
         consume(w2, sc2, base + 8 * U);
     }
-    lm_finish(a, wave_max_key(best), bkey, &last_block);
+    lm_finish(a, t_begin, wave_max_key(best), bkey, &last_block);
 }
 
 typedef void (*GemvKernel)(GemvArgs);
@@ -1072,10 +1089,12 @@ int mdx_launch_norm_gemv(const float* hidden, const float* norm_w, float eps, co
     return launch_gemv(kind, a, rw, 0, stream);
 }
 
-int mdx_launch_embed_norm_gemv(const mdx_state* state, const float* emb_table, const float* emb_in,
-                               int vocab, float* hidden, const float* norm_w, float eps,
-                               const mdx_wdesc* w, float* out, void* stream) {
+int mdx_launch_embed_norm_gemv(const mdx_state* state, mdx_state* dev_state, mdx_host_res* res,
+                               const float* emb_table, const float* emb_in, int vocab, float* hidden,
+                               const float* norm_w, float eps, const mdx_wdesc* w, float* out, void* stream) {
     GemvArgs a = base_args(w);
+    a.st_copy = dev_state;
+    a.res = res;
     a.xmode = XM_EMBED;
     a.st_in = state;
     a.emb_table = emb_table;
@@ -1124,8 +1143,9 @@ size_t mdx_lmhead_scratch_bytes(void) { return sizeof(LmScratch); }
 
 int mdx_launch_lmhead(const float* hidden, const float* norm_w, float eps, const mdx_wdesc* w,
                       float* logits, void* scratch, mdx_state* state, int* out_tokens, int advance,
-                      void* stream) {
+                      mdx_host_res* res, void* stream) {
     GemvArgs a = base_args(w);
+    a.res = res;
     a.xmode = XM_NORM;
     a.xf32 = hidden;
     a.norm_w = norm_w;

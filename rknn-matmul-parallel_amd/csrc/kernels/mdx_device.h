@@ -41,6 +41,18 @@ typedef struct {
     int pad[3];
 } mdx_state;
 
+/* What a step leaves in pinned memory for the host (which clears it first).
+ * Times are ticks of the device's wall clock (mdxrt_clock_khz). */
+typedef struct {
+    int argmax;
+    int timeout;                    /* 1 when a wait of the one-launch step timed out */
+    int done;                       /* set last, by mdxrt_signal or the lm_head */
+    int pad;
+    unsigned long long t_start;     /* the step's first kernel */
+    unsigned long long t_layers;    /* end of the one launch, or start of the lm_head kernel */
+    unsigned long long t_end;       /* when done was set */
+} mdx_host_res;
+
 /* ---- runtime wrappers (mdx_rt.hip) ---- */
 int mdxrt_device_count(void);
 const char* mdxrt_last_error(void);
@@ -69,15 +81,18 @@ int mdxrt_graph_destroy(void* exec);
 int mdxrt_event_create(void** ev);
 int mdxrt_event_destroy(void* ev);
 int mdxrt_event_record(void* ev, void* stream);
+int mdxrt_event_sync(void* ev);
 int mdxrt_event_elapsed_ms(void* start, void* stop, float* ms);
 /* Copy by a kernel between device memory and pinned host memory (16-byte
  * addresses and size). */
 int mdxrt_copy16(void* dst, const void* src, size_t bytes, void* stream);
-/* mdxrt_signal stores 1 in the pinned word *flag once everything before it on
- * the stream is complete; mdxrt_wait returns when it is there.  The caller
- * clears the word before it issues the work. */
-int mdxrt_signal(int* flag, void* stream);
+/* mdxrt_signal stores 1 in the pinned word *flag (and the wall clock in *t
+ * when given) once everything before it on the stream is complete; mdxrt_wait
+ * returns when it is there.  The caller clears the word before it issues the
+ * work. */
+int mdxrt_signal(int* flag, unsigned long long* t, void* stream);
 int mdxrt_wait(int* flag, void* stream);
+int mdxrt_clock_khz(void);
 /* Fill `n` 32-bit words with `value` on the stream (a kernel, never a
  * memset node, so it is safe inside captured graphs). */
 int mdxrt_fill_u32(void* dst, uint32_t value, size_t n, void* stream);
@@ -92,10 +107,12 @@ int mdx_launch_norm_gemv(const float* hidden, const float* norm_w, float eps,
 
 /* First projection of a step: the input row is embeddings[state->token]
  * (state->mode 0) or emb_in (mode 1); it is copied to hidden[d] and then
- * RMSNorm + projection as mdx_launch_norm_gemv, storing y fp32. */
-int mdx_launch_embed_norm_gemv(const mdx_state* state, const float* emb_table, const float* emb_in,
-                               int vocab, float* hidden, const float* norm_w, float eps,
-                               const mdx_wdesc* w, float* out, void* stream);
+ * RMSNorm + projection as mdx_launch_norm_gemv, storing y fp32.  With
+ * dev_state, state (and emb_in) are in pinned memory and state is copied to
+ * dev_state for the kernels that follow; res (may be NULL): t_start. */
+int mdx_launch_embed_norm_gemv(const mdx_state* state, mdx_state* dev_state, mdx_host_res* res,
+                               const float* emb_table, const float* emb_in, int vocab, float* hidden,
+                               const float* norm_w, float eps, const mdx_wdesc* w, float* out, void* stream);
 
 /* y = fp16 x . W^T (x scale); out[n] += y[n] (residual add, fp32). */
 int mdx_launch_gemv_add(const uint16_t* x16, const mdx_wdesc* w, float* out, void* stream);
@@ -130,11 +147,13 @@ int mdx_launch_attn_decode(const mdx_state* state, const float* qkv, const float
  * when out_tokens != NULL and advances state->pos by `advance`.
  * w->kind: MDX_W_I8 (fp16 activations, the NPU path), MDX_W_F16 with fp32
  * activations (the CPU fp16 GEMV), MDX_W_F32 (fp32 rows).  scratch:
- * mdx_lmhead_scratch_bytes() zero bytes (left zero by the kernel). */
+ * mdx_lmhead_scratch_bytes() zero bytes (left zero by the kernel).  res (may
+ * be NULL): argmax and t_layers, the time the kernel started; logits may be
+ * pinned memory. */
 size_t mdx_lmhead_scratch_bytes(void);
 int mdx_launch_lmhead(const float* hidden, const float* norm_w, float eps, const mdx_wdesc* w,
                       float* logits, void* scratch, mdx_state* state, int* out_tokens, int advance,
-                      void* stream);
+                      mdx_host_res* res, void* stream);
 /* state->pos += advance (prefill-mode steps). */
 int mdx_launch_advance(mdx_state* state, int advance, void* stream);
 
@@ -172,7 +191,7 @@ typedef struct {
     long long layer_stride;
     long long kv_stride;
     const float* emb_table;            /* [vocab][d] fp32 */
-    const float* emb_in;               /* [d], used when state->mode == 1 */
+    const float* emb_in;               /* [d] in pinned memory, used in mode 1 */
     const float* cos_t;
     const float* sin_t;
     const float* final_norm;
@@ -198,8 +217,7 @@ typedef struct {
     float* logits_host;                /* optional (head only, vocab <= 256 * 1024): the
                                           logits written to this mapped host buffer instead
                                           of logits */
-    int* res_host;                     /* optional mapped host words: [0] <- the argmax,
-                                          [1] <- 1 when a wait timed out */
+    mdx_host_res* res_host;            /* optional: argmax, timeout, t_start and t_layers */
     void* xbl;                         /* optional: cacheable words (mdx_persist_xbuf_bytes(),
                                           zeroed) for the exchanges among one KV head's
                                           workgroups, which share an XCD; NULL: those go

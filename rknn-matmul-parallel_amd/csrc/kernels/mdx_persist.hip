@@ -124,7 +124,7 @@ struct PArgs {
     int in_args;                // 1: pos, token, mode from the three fields below, not st
     int in_pos, in_token, in_mode;
     float* logits_host;         // optional mapped host buffer for the logits (instead of logits)
-    int* res_host;              // optional mapped host words: [0] the argmax, [1] set on a timeout
+    mdx_host_res* res_host;     // optional: argmax, timeout, t_start, t_layers
     unsigned* xbl;              // optional cacheable words for the per-head exchanges
 };
 
@@ -509,7 +509,13 @@ __global__ __launch_bounds__(NT) void k_persist_step(PArgs a) {
     // the result words without a copy
     auto flag_timeout = [&]() {
         __hip_atomic_store(&a.st->pad[1], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (a.res_host) __hip_atomic_store(&a.res_host[1], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        if (a.res_host) __hip_atomic_store(&a.res_host->timeout, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    };
+    const unsigned long long t_start = a.res_host ? wall_clock64() : 0;
+    auto times = [&]() {
+        if (!a.res_host) return;
+        a.res_host->t_start = t_start;
+        a.res_host->t_layers = wall_clock64();
     };
     bool dead = false;
     const unsigned spin_lim = a.spin_limit;
@@ -1246,7 +1252,8 @@ __global__ __launch_bounds__(NT) void k_persist_step(PArgs a) {
             }
             st->pos = pos + a.advance;
             if (dead) flag_timeout();
-            if (a.res_host) __hip_atomic_store(&a.res_host[0], res, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            if (a.res_host) __hip_atomic_store(&a.res_host->argmax, res, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            times();
             __hip_atomic_store(xb + W_CTRL, E + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
         if (a.logits_host) logits_out();
@@ -1255,6 +1262,7 @@ __global__ __launch_bounds__(NT) void k_persist_step(PArgs a) {
         if (dead && t == 0) flag_timeout();
         if (b == 0 && t == 0) {
             a.st->pos = pos + a.advance;
+            times();
             __hip_atomic_store(xb + W_CTRL, E + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     }

@@ -42,8 +42,10 @@ __global__ __launch_bounds__(256) void k_copy16(uint4* dst, const uint4* src, si
 
 // The word the host polls (mdxrt_wait): everything before this kernel on its
 // stream is complete, its stores to host memory included.
-__global__ void k_signal(int* flag) {
-    if (threadIdx.x == 0) __hip_atomic_store(flag, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+__global__ void k_signal(int* flag, unsigned long long* t) {
+    if (threadIdx.x != 0) return;
+    if (t) *t = wall_clock64();
+    __hip_atomic_store(flag, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 }  // namespace
@@ -253,6 +255,11 @@ int mdxrt_event_record(void* ev, void* stream) {
     return 0;
 }
 
+int mdxrt_event_sync(void* ev) {
+    MDX_CHECK(hipEventSynchronize((hipEvent_t)ev), "hipEventSynchronize");
+    return 0;
+}
+
 int mdxrt_event_elapsed_ms(void* start, void* stop, float* ms) {
     MDX_CHECK(hipEventSynchronize((hipEvent_t)stop), "hipEventSynchronize");
     MDX_CHECK(hipEventElapsedTime(ms, (hipEvent_t)start, (hipEvent_t)stop), "hipEventElapsedTime");
@@ -270,8 +277,8 @@ int mdxrt_copy16(void* dst, const void* src, size_t bytes, void* stream) {
     return 0;
 }
 
-int mdxrt_signal(int* flag, void* stream) {
-    k_signal<<<dim3(1), dim3(64), 0, (hipStream_t)stream>>>(flag);
+int mdxrt_signal(int* flag, unsigned long long* t, void* stream) {
+    k_signal<<<dim3(1), dim3(64), 0, (hipStream_t)stream>>>(flag, t);
     MDX_CHECK(hipGetLastError(), "k_signal");
     return 0;
 }
@@ -292,6 +299,14 @@ int mdxrt_wait(int* flag, void* stream) {
     if (__atomic_load_n(flag, __ATOMIC_ACQUIRE)) return 0;
     std::snprintf(g_last_error, sizeof g_last_error, "mdxrt_wait: the stream is idle but did not signal");
     return -4;
+}
+
+int mdxrt_clock_khz(void) {
+    int dev = 0, khz = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev) != hipSuccess || khz <= 0)
+        khz = 100000;
+    return khz;
 }
 
 int mdxrt_fill_u32(void* dst, uint32_t value, size_t n, void* stream) {
