@@ -21,13 +21,16 @@ using namespace mdx;
 
 namespace {
 
+typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
+
 constexpr int kKT = 64;            // k per LDS stage
 constexpr int kRun = 4;            // stages per partial sum
 constexpr int kStageChunks = kKT / 8;   // 16-byte chunks per LDS row
 
-// Where the tile's 16-byte chunk of row r goes: chunks are permuted within the
-// row by the row index, so the 16 rows of an MFMA fragment read spread over
-// the banks without padding.
+// Where a tile's 16-byte chunk of row r goes: chunks are permuted within the
+// row by the row index, so the rows of an MFMA fragment read spread over the
+// banks without padding (padded rows instead: M = 2000 projections 141 -> 146
+// us a layer).
 __device__ __forceinline__ int lds_chunk(int row, int chunk) {
     return row * kStageChunks + (chunk ^ (row & 7));
 }
@@ -193,8 +196,12 @@ __global__ __launch_bounds__(256, 2) void k_long_gemm(LongArgs a) {
     const int s0 = split * a.per_split, s1 = min(nst_all, s0 + a.per_split);
     const size_t row_bytes = KIND == MDX_W_F16 ? (size_t)a.K * 2 : (KIND == MDX_W_I8 ? (size_t)a.K : (size_t)a.K / 2);
 
-    // this thread's loads: rows past the edge repeat the last row (their
-    // results are not stored)
+    // This thread's loads.  None is conditional, so the compiler can count the
+    // ones in flight and waits for no younger stage than the one it needs (a
+    // load under a branch makes it wait for all: M = 203, K = 1024 took 1 us a
+    // stage whatever PD).  Rows past the edge repeat the last row (their
+    // results are not stored), stages past the last repeat it, and k past K
+    // repeat the row's last load and become zeros on their way to LDS.
     const uint16_t* xp[XU];
     int xk[XU], xl[XU];
 #pragma unroll
@@ -202,7 +209,7 @@ __global__ __launch_bounds__(256, 2) void k_long_gemm(LongArgs a) {
         const int u = tid + 256 * i, row = u / kStageChunks, ch = u % kStageChunks;
         xk[i] = 8 * ch;
         xl[i] = lds_chunk(row, ch);
-        xp[i] = a.x16 + (size_t)min(tm * BM + row, a.M - 1) * a.K + 8 * ch;
+        xp[i] = a.x16 + (size_t)min(tm * BM + row, a.M - 1) * a.K;
     }
     const uint8_t* wp[WU];
     int wk[WU], wr[WU];
@@ -211,28 +218,33 @@ __global__ __launch_bounds__(256, 2) void k_long_gemm(LongArgs a) {
         const int u = min(tid + 256 * i, WUN - 1), row = u / UPR, ch = u % UPR;
         wk[i] = KPU * ch;
         wr[i] = row;
-        wp[i] = a.w + (size_t)min(long_row<BN>(tn, row, SWIGLU, a.N), a.N - 1) * row_bytes + (size_t)ch * 16;
+        wp[i] = a.w + (size_t)min(long_row<BN>(tn, row, SWIGLU, a.N), a.N - 1) * row_bytes;
     }
-    uint4 xv[PD][XU], wv[PD][WU];
-    // K is a multiple of 32, so no load straddles it; those past it are zeros
-    auto load = [&](int d, int st) {
-        const int k0 = st * kKT;
+    u32x4_t xv[PD][XU], wv[PD][WU];
+    auto load = [&](int d, int st) __attribute__((always_inline)) {
+        const int k0 = min(st, s1 - 1) * kKT;
 #pragma unroll
         for (int i = 0; i < XU; i++)
-            xv[d][i] = k0 + xk[i] < a.K ? *reinterpret_cast<const uint4*>(xp[i] + k0) : make_uint4(0u, 0u, 0u, 0u);
+            xv[d][i] = *reinterpret_cast<const u32x4_t*>(xp[i] + (unsigned)min(k0 + xk[i], a.K - 8));
 #pragma unroll
-        for (int i = 0; i < WU; i++)
-            wv[d][i] = k0 + wk[i] < a.K ? *reinterpret_cast<const uint4*>(wp[i] + (size_t)st * (16 * UPR))
-                                        : make_uint4(0u, 0u, 0u, 0u);
+        for (int i = 0; i < WU; i++) {
+            const unsigned k = (unsigned)min(k0 + wk[i], a.K - KPU);
+            wv[d][i] = *reinterpret_cast<const u32x4_t*>(wp[i] + (KIND == MDX_W_F16 ? 2 * k : KIND == MDX_W_I8 ? k : k / 2));
+        }
     };
-    auto stash = [&](int d, int buf) {
+    auto stash = [&](int d, int buf, int st) __attribute__((always_inline)) {
+        if ((st + 1) * kKT > a.K) {       // K ends inside this stage
 #pragma unroll
-        for (int i = 0; i < XU; i++) xs[buf][xl[i]] = xv[d][i];
+            for (int i = 0; i < XU; i++)
+                if (st * kKT + xk[i] >= a.K) xv[d][i] = u32x4_t{0u, 0u, 0u, 0u};
+        }
+#pragma unroll
+        for (int i = 0; i < XU; i++) xs[buf][xl[i]] = __builtin_bit_cast(uint4, xv[d][i]);
 #pragma unroll
         for (int i = 0; i < WU; i++) {
             if (WUN % 256 != 0 && tid + 256 * i >= WUN) break;
             half8_t b[KPU / 8];
-            widen_b<KIND>(wv[d][i], b);
+            widen_b<KIND>(__builtin_bit_cast(uint4, wv[d][i]), b);
 #pragma unroll
             for (int s = 0; s < KPU / 8; s++)
                 ws[buf][lds_chunk(wr[i], wk[i] / 8 + s)] = __builtin_bit_cast(uint4, b[s]);
@@ -241,7 +253,7 @@ __global__ __launch_bounds__(256, 2) void k_long_gemm(LongArgs a) {
 
     // sums of kRun stages (256 k) are added to a second set: one running sum
     // over all of K loses precision (K = 3072: 3.5e-7 off the exact products'
-    // sum in the 2-norm, against PREC so)
+    // sum in the 2-norm, against 1.2e-7 so)
     float4_t acc[NT][MT], tot[NT][MT];
 #pragma unroll
     for (int t = 0; t < NT; t++)
@@ -249,10 +261,9 @@ __global__ __launch_bounds__(256, 2) void k_long_gemm(LongArgs a) {
         for (int j = 0; j < MT; j++) acc[t][j] = tot[t][j] = float4_t{0.f, 0.f, 0.f, 0.f};
 
 #pragma unroll
-    for (int d = 0; d < PD; d++)
-        if (s0 + d < s1) load(d, s0 + d);
-    stash(0, 0);
-    if (s0 + PD < s1) load(0, s0 + PD);
+    for (int d = 0; d < PD; d++) load(d, s0 + d);
+    stash(0, 0, s0);
+    load(0, s0 + PD);
     __syncthreads();
     for (int sb = s0; sb < s1; sb += PD) {
 #pragma unroll
@@ -260,6 +271,11 @@ __global__ __launch_bounds__(256, 2) void k_long_gemm(LongArgs a) {
             const int st = sb + d;
             if (st >= s1) break;
             const int buf = (st - s0) & 1;
+            // the next stage's LDS writes and a later one's loads are issued
+            // before this one's products
+            const int dn = (d + 1) % PD;
+            stash(dn, buf ^ 1, st + 1);
+            load(dn, st + 1 + PD);
 #pragma unroll
             for (int s = 0; s < 2; s++) {
                 half8_t xb[MT];
@@ -282,11 +298,6 @@ __global__ __launch_bounds__(256, 2) void k_long_gemm(LongArgs a) {
                         tot[t][j] += acc[t][j];
                         acc[t][j] = float4_t{0.f, 0.f, 0.f, 0.f};
                     }
-            }
-            if (st + 1 < s1) {
-                const int dn = (d + 1) % PD;
-                stash(dn, buf ^ 1);
-                if (st + 1 + PD < s1) load(dn, st + 1 + PD);
             }
             __syncthreads();
         }
@@ -361,22 +372,35 @@ __global__ __launch_bounds__(256, 2) void k_long_gemm(LongArgs a) {
 // ---- attention ------------------------------------------------------------------
 //
 // Block = one KV head x 64 query rows (64/G consecutive positions x the G
-// heads of the group), 16 rows per wave; K/V tiles of 64 positions staged in
-// LDS (V transposed), the next tile in registers meanwhile.  S^T = K . Q^T,
+// heads of the group), 16 rows per wave and two groups of four waves, which
+// take alternate K/V tiles of 64 positions and are merged at the end: the
+// causal rows make the last blocks twice as long as the average one, and
+// nothing else is left to run beside them, so a block's own length is what
+// counts (one group, two blocks per CU: 67 us at M = 2000, 55 with two).
+// Tiles are staged in LDS (V transposed), the group's next one in registers
+// meanwhile.  S^T = K . Q^T,
 // so a lane holds scores of one query row and its running maximum and sum are
 // its own; P^T is then already the B operand of O^T = V^T . P^T (the k order
 // of that product is the order in which a lane holds its scores).
 //
 // Queries and probabilities are fp32: each goes in as the sum of two fp16
 // values (22 bits), the queries scaled per row so that neither part leaves the
-// fp16 range, the probabilities by 2^14.
+// fp16 range, the probabilities by 2^6 relative to a reference score.
+//
+// The vector unit is what bounds it (at M = 2000 the longest block's tile took
+// 2.9 us with expf and a rescale per tile): the exponentials are v_exp_f32 of
+// one fma (the row's scale, the softmax scale and log2 e are one factor, as
+// exact as the fp32 score), the reference score only moves, and the sums are
+// only rescaled, when a row's maximum has outgrown it by 2^8, and addresses are
+// clamped instead of values selected.  16 query heads of 128 over 8 KV heads,
+// M = 2000: 92 -> 67 us by these.
 //
 // Infinities and NaN: scores that come out as NaN are recomputed in fp32 (an
 // infinite key times the two parts of a query may be inf - inf), and a V tile
 // that holds any takes the products of its own positions only, in fp32, so
 // that a position beyond a row's own never reaches that row.
 typedef unsigned short u16x2_t __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ uint32_t max_exp(uint32_t m, uint4 v) {
+__device__ __forceinline__ uint32_t max_exp(uint32_t m, u32x4_t v) {
     const uint32_t w[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
     for (int i = 0; i < 4; i++)
@@ -386,14 +410,26 @@ __device__ __forceinline__ uint32_t max_exp(uint32_t m, uint4 v) {
 }
 __device__ __forceinline__ bool exp_nonfinite(uint32_t m) { return (m & 0xffffu) >= 0x7c00u || (m >> 16) >= 0x7c00u; }
 
-// fp32 as the sum of two fp16 values.
-__device__ __forceinline__ void split16(float v, _Float16& hi, _Float16& lo) {
-    hi = (_Float16)v;
-    lo = (_Float16)(v - (float)hi);
+// fp32 pairs as the sums of two fp16 values: the first part rounds towards
+// zero (one instruction for both), the second holds the remainder.
+__device__ __forceinline__ void split16(float a, float b, half2_t& hi, half2_t& lo) {
+    hi = __builtin_bit_cast(half2_t, __builtin_amdgcn_cvt_pkrtz(a, b));
+    lo = half2_t{(_Float16)(a - (float)hi.x), (_Float16)(b - (float)hi.y)};
+}
+__device__ __forceinline__ void split16(const float (&v)[8], half8_t& hi, half8_t& lo) {
+#pragma unroll
+    for (int e = 0; e < 8; e += 2) {
+        half2_t h, l;
+        split16(v[e], v[e + 1], h, l);
+        hi[e] = h.x;
+        hi[e + 1] = h.y;
+        lo[e] = l.x;
+        lo[e + 1] = l.y;
+    }
 }
 
 template <int HD, int G>
-__global__ __launch_bounds__(256, 2) void k_attn_long(int pos0, int M, const float* __restrict__ q,
+__global__ __launch_bounds__(512, 2) void k_attn_long(int pos0, int M, const float* __restrict__ q,
                                                       const uint16_t* __restrict__ kc,
                                                       const uint16_t* __restrict__ vc, int nkv, int n_tb,
                                                       uint16_t* __restrict__ out16) {
@@ -406,11 +442,15 @@ __global__ __launch_bounds__(256, 2) void k_attn_long(int pos0, int M, const flo
     constexpr int KU = KB * (HD / 8) / 256;        // K loads per thread
     constexpr int VUN = (KB / 4) * (HD / 8);       // V units: 4 keys x 8 dims
     constexpr int VU = (VUN + 255) / 256;
-    // the K tile, or the fp32 probabilities of a non-finite V tile (64 rows x KB)
-    __shared__ uint4 ks[KB * KS > 16 * KB ? KB * KS : 16 * KB];
-    __shared__ uint4 vs[HD * VS];
+    // a group's K tile, or the fp32 probabilities of a non-finite V tile (64 rows x KB)
+    constexpr int KN = KB * KS > 16 * KB ? KB * KS : 16 * KB;
+    constexpr int MN = (4 * DT + 2) * 256 / 4;     // uint4 of a group's sums in the merge
+    static_assert(2 * (KN + HD * VS) >= MN, "the merge fits the tiles");
+    __shared__ uint4 lds[2 * (KN + HD * VS)];
 
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int grp = threadIdx.x >> 8, tid = threadIdx.x & 255, wave = tid >> 6, lane = tid & 63;
+    uint4* const ks = lds + grp * (KN + HD * VS);
+    uint4* const vs = ks + KN;
     const int g = lane >> 4, c16 = lane & 15;
     const int kvh = blockIdx.x % nkv;
     const int t0 = (n_tb - 1 - blockIdx.x / nkv) * TB;   // the longest blocks first
@@ -423,31 +463,32 @@ __global__ __launch_bounds__(256, 2) void k_attn_long(int pos0, int M, const flo
     const float* qrow = q + ((size_t)(tv ? t : M - 1) * nq + hq) * HD;
 
     // K/V tile loads of this thread
-    const uint16_t* kp = kc + (size_t)kvh * HD;
-    const uint16_t* vp = vc + (size_t)kvh * HD;
-    uint4 kr[KU], vr[VU][4];
-    auto load = [&](int p0) {
+    u32x4_t kr[KU], vr[VU][4];
+    auto load = [&](int p0) __attribute__((always_inline)) {
+        // positions past the block's last repeat it (their scores are masked)
+        const int pb = min(p0, Lmax - 1), last = Lmax - 1 - pb;
+        const uint16_t* kp = kc + (size_t)pb * kvd + kvh * HD;
+        const uint16_t* vp = vc + (size_t)pb * kvd + kvh * HD;
 #pragma unroll
         for (int i = 0; i < KU; i++) {
             const int u = tid + 256 * i, key = u / (HD / 8), ch = u % (HD / 8);
-            kr[i] = p0 + key < Lmax ? *reinterpret_cast<const uint4*>(kp + (size_t)(p0 + key) * kvd + 8 * ch)
-                                    : make_uint4(0u, 0u, 0u, 0u);
+            kr[i] = *reinterpret_cast<const u32x4_t*>(kp + (unsigned)(min(key, last) * kvd + 8 * ch));
         }
 #pragma unroll
         for (int i = 0; i < VU; i++) {
             const int u = tid + 256 * i, kg = u % (KB / 4), db = u / (KB / 4);
+            if (VUN % 256 != 0 && db >= HD / 8) break;
 #pragma unroll
             for (int j = 0; j < 4; j++)
-                vr[i][j] = db < HD / 8 && p0 + 4 * kg + j < Lmax
-                               ? *reinterpret_cast<const uint4*>(vp + (size_t)(p0 + 4 * kg + j) * kvd + 8 * db)
-                               : make_uint4(0u, 0u, 0u, 0u);
+                vr[i][j] = *reinterpret_cast<const u32x4_t*>(vp + (unsigned)(min(4 * kg + j, last) * kvd + 8 * db));
         }
     };
-    load(0);
+    load(grp * KB);
 
-    // the query row as fp16 pairs, scaled by 2^e to a maximum in [2^14, 2^15)
+    // the query row as fp16 pairs, scaled by 2^e to a maximum in [2^14, 2^15);
+    // a score times c is its exponent in base 2
     half8_t qh[DS], ql[DS];
-    float qscale;
+    float up, c;
     {
         float qv[DS][8], mx = 0.0f;
 #pragma unroll
@@ -465,30 +506,29 @@ __global__ __launch_bounds__(256, 2) void k_attn_long(int pos0, int M, const flo
             ex = 14 - ilogbf(mx);
             ex = ex > 100 ? 100 : ex;
         }
-        const float up = ldexpf(1.0f, ex);
-        qscale = ldexpf(1.0f / sqrtf((float)HD), -ex);
+        up = ldexpf(1.0f, ex);
+        c = ldexpf(1.44269504088896340736f / sqrtf((float)HD), -ex);
 #pragma unroll
-        for (int s = 0; s < DS; s++)
+        for (int s = 0; s < DS; s++) {
 #pragma unroll
-            for (int e = 0; e < 8; e++) {
-                _Float16 h, l;
-                split16(qv[s][e] * up, h, l);
-                qh[s][e] = h;
-                ql[s][e] = l;
-            }
+            for (int e = 0; e < 8; e++) qv[s][e] *= up;
+            split16(qv[s], qh[s], ql[s]);
+        }
     }
 
     float4_t o[DT];
 #pragma unroll
     for (int d = 0; d < DT; d++) o[d] = float4_t{0.f, 0.f, 0.f, 0.f};
-    float runM = -INFINITY, runL = 0.0f;
+    float ref = -INFINITY, runL = 0.0f;       // ref: base-2 exponent of the reference score
 
-    for (int p0 = 0; p0 < Lmax; p0 += KB) {
+    // the groups' tiles of a round; the last one of group 1 may be all masked
+    for (int pr0 = 0; pr0 < Lmax; pr0 += 2 * KB) {
+        const int p0 = pr0 + grp * KB;
         uint32_t vmax = 0;
 #pragma unroll
         for (int i = 0; i < KU; i++) {
             const int u = tid + 256 * i;
-            ks[(u / (HD / 8)) * KS + u % (HD / 8)] = kr[i];
+            ks[(u / (HD / 8)) * KS + u % (HD / 8)] = __builtin_bit_cast(uint4, kr[i]);
         }
 #pragma unroll
         for (int i = 0; i < VU; i++) {
@@ -514,12 +554,13 @@ __global__ __launch_bounds__(256, 2) void k_attn_long(int pos0, int M, const flo
             }
         }
         const bool slow = __syncthreads_or(exp_nonfinite(vmax));
-        if (p0 + KB < Lmax) load(p0 + KB);
+        load(p0 + 2 * KB);
 
-        // scores: s[kt][i] = key p0 + 16 kt + 4 g + i, then their exponentials
+        // scores: s[kt][i] = key p0 + 16 kt + 4 g + i, then 2^6 times their
+        // exponentials relative to the reference
         float4_t s[KB / 16];
-        float alpha, ls, mx;
-        auto softmax = [&]() {
+        float ls, next;
+        auto softmax = [&]() __attribute__((always_inline)) {
             if (p0 + KB > pos0 + t0 + 1) {      // some row of the block ends inside this tile
 #pragma unroll
                 for (int kt = 0; kt < KB / 16; kt++)
@@ -527,19 +568,19 @@ __global__ __launch_bounds__(256, 2) void k_attn_long(int pos0, int M, const flo
                     for (int i = 0; i < 4; i++)
                         if (p0 + 16 * kt + 4 * g + i >= L) s[kt][i] = -INFINITY;
             }
-            mx = -INFINITY;
+            float mx = -INFINITY;
 #pragma unroll
             for (int kt = 0; kt < KB / 16; kt++)
                 mx = fmaxf(mx, fmaxf(fmaxf(s[kt][0], s[kt][1]), fmaxf(s[kt][2], s[kt][3])));
-            mx = fmaxf(runM, rows_max4(mx));
-            const float ref = mx == -INFINITY ? 0.0f : mx;   // no score above -inf yet: p = 0
-            alpha = expf(runM - ref);
+            const float m2 = rows_max4(mx) * c;
+            next = m2 > ref + 8.0f ? m2 : ref;          // (the first score: ref is -inf)
+            const float off = next == -INFINITY ? 0.0f : 6.0f - next;
             ls = 0.0f;
 #pragma unroll
             for (int kt = 0; kt < KB / 16; kt++)
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
-                    s[kt][i] = expf(s[kt][i] - ref);
+                    s[kt][i] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[kt][i], c, off));
                     ls = ls + s[kt][i];
                 }
         };
@@ -552,13 +593,10 @@ __global__ __launch_bounds__(256, 2) void k_attn_long(int pos0, int M, const flo
                 s[kt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(k8, qh[d], s[kt], 0, 0, 0);
                 s[kt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(k8, ql[d], s[kt], 0, 0, 0);
             }
-#pragma unroll
-            for (int i = 0; i < 4; i++) s[kt][i] = s[kt][i] * qscale;
         }
         softmax();
         if (__any(ls != ls)) {
             const uint16_t* kb = reinterpret_cast<const uint16_t*>(ks);
-            const float sc = 1.0f / sqrtf((float)HD);
 #pragma unroll
             for (int kt = 0; kt < KB / 16; kt++)
 #pragma unroll
@@ -567,27 +605,27 @@ __global__ __launch_bounds__(256, 2) void k_attn_long(int pos0, int M, const flo
                     float sum = 0.0f;
 #pragma unroll 1
                     for (int d = 0; d < HD; d++) sum = sum + qrow[d] * f16_bits_to_f32(kk[d]);
-                    s[kt][i] = sum * sc;
+                    s[kt][i] = sum * up;
                 }
             softmax();
         }
-        runM = mx;
-        runL = runL * alpha + ls;
+        if (__any(next != ref)) {
+            const float alpha = next == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(ref - next);
+            runL = runL * alpha;
 #pragma unroll
-        for (int d = 0; d < DT; d++)
+            for (int d = 0; d < DT; d++)
 #pragma unroll
-            for (int i = 0; i < 4; i++) o[d][i] = o[d][i] * alpha;
+                for (int i = 0; i < 4; i++) o[d][i] = o[d][i] * alpha;
+            ref = next;
+        }
+        runL = runL + ls;
         if (!slow) {
 #pragma unroll
             for (int pr = 0; pr < KB / 32; pr++) {
+                const float pv[8] = {s[2 * pr][0], s[2 * pr][1], s[2 * pr][2], s[2 * pr][3],
+                                     s[2 * pr + 1][0], s[2 * pr + 1][1], s[2 * pr + 1][2], s[2 * pr + 1][3]};
                 half8_t ph, pl;
-#pragma unroll
-                for (int e = 0; e < 8; e++) {
-                    _Float16 h, l;
-                    split16(s[2 * pr + e / 4][e % 4] * 16384.0f, h, l);
-                    ph[e] = h;
-                    pl[e] = l;
-                }
+                split16(pv, ph, pl);
 #pragma unroll
                 for (int d = 0; d < DT; d++) {
                     const half8_t v8 = __builtin_bit_cast(half8_t, vs[(16 * d + c16) * VS + 4 * pr + g]);
@@ -607,7 +645,7 @@ __global__ __launch_bounds__(256, 2) void k_attn_long(int pos0, int M, const flo
 #pragma unroll 1
             for (int key = 0; key < KB; key++) {
                 if (p0 + key >= L) break;
-                const float p = pf[c16 * KB + key] * 16384.0f;
+                const float p = pf[c16 * KB + key];
                 const int off = 32 * (key >> 5) + 8 * ((key >> 2) & 3) + 4 * ((key >> 4) & 1) + (key & 3);
 #pragma unroll
                 for (int d = 0; d < DT; d++)
@@ -618,8 +656,27 @@ __global__ __launch_bounds__(256, 2) void k_attn_long(int pos0, int M, const flo
         }
         __syncthreads();                    // the tile is rewritten
     }
-    if (!tv) return;
-    const float l = rows_sum4(runL) * 16384.0f;
+    // group 1's sums, brought to a common reference
+    float* const mg = reinterpret_cast<float*>(lds) + tid;
+    if (grp == 1) {
+#pragma unroll
+        for (int d = 0; d < DT; d++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) mg[(4 * d + i) * 256] = o[d][i];
+        mg[4 * DT * 256] = ref;
+        mg[(4 * DT + 1) * 256] = runL;
+    }
+    __syncthreads();
+    if (grp == 1 || !tv) return;
+    const float ref1 = mg[4 * DT * 256], top = fmaxf(ref, ref1);
+    // (a reference of -inf: no score above -inf, sums of zero or NaN)
+    const float a0 = ref == top ? 1.0f : __builtin_amdgcn_exp2f(ref - top);
+    const float a1 = ref1 == top ? 1.0f : __builtin_amdgcn_exp2f(ref1 - top);
+#pragma unroll
+    for (int d = 0; d < DT; d++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) o[d][i] = o[d][i] * a0 + mg[(4 * d + i) * 256] * a1;
+    const float l = rows_sum4(runL * a0 + mg[(4 * DT + 1) * 256] * a1);
     uint16_t* dst = out16 + ((size_t)t * nq + hq) * HD + 4 * g;
 #pragma unroll
     for (int d = 0; d < DT; d++) {
@@ -771,7 +828,7 @@ int mdx_launch_long_attn(int pos0, const float* q, int M, const uint16_t* k_cach
     dim3 grid((unsigned)(n_tb * nkv));
 #define MDX_LATTN(HD_, G_)                                                                                 \
     if (hd == HD_ && G == G_) {                                                                            \
-        hipLaunchKernelGGL((k_attn_long<HD_, G_>), grid, dim3(256), 0, (hipStream_t)stream, pos0, M, q,    \
+        hipLaunchKernelGGL((k_attn_long<HD_, G_>), grid, dim3(512), 0, (hipStream_t)stream, pos0, M, q,    \
                            k_cache, v_cache, nkv, n_tb, out16);                                            \
         return hipGetLastError() == hipSuccess ? 0 : -4;                                                   \
     }
