@@ -716,21 +716,51 @@ struct AttnArgs {
     uint16_t* vc;
     int nkv;
     int max_splits;
-    int chunk_cap;
     float* part;              // [nkv][max_splits][G][hd + 4]
     unsigned int* done;       // [nkv], zero between launches
     uint16_t* out16;          // [nq*hd]
 };
 
 // Splits of up to kAttnChunk positions (more when L exceeds max_splits of
-// them): fewer split records to merge, and a block's tiles are requested
-// together (k_attn_decode issues its first kAttnPf tiles before anything else).
-constexpr int kAttnChunk = 64, kAttnPf = 4;
+// them); a single one, which needs no records and no merge (about 2.5 us a
+// layer), for as long as that is less than what its positions take: 256 at
+// head_dim 64 (8 layers at 247 positions: 164 us a token, 172 in two splits),
+// 128 at the others (128: 276 us, 263 in two; 256: 294, 250 in two).
+constexpr int kAttnChunk = 128;
+template <int HD> constexpr int kAttnOne = HD == 64 ? 256 : kAttnChunk;
+template <int HD>
 __device__ __forceinline__ void attn_plan(int L, int max_splits, int& splits, int& chunk) {
-    int s = (L + kAttnChunk - 1) / kAttnChunk;
+    int s = L <= kAttnOne<HD> ? 1 : (L + kAttnChunk - 1) / kAttnChunk;
     if (s > max_splits) s = max_splits;
     chunk = (L + s - 1) / s;
     splits = (L + chunk - 1) / chunk;
+}
+
+// The lanes that differ in one bit of the position slot (lane bit O).
+template <int O>
+__device__ __forceinline__ float max_step(float v) {
+    if constexpr (O == 32) {
+        const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+        return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+    } else if constexpr (O == 16) {
+        const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+        return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+    } else {
+        return fmaxf(v, partner<O>(v));
+    }
+}
+// Sum over the LP lanes of a position.
+template <int LP>
+__device__ __forceinline__ float pos_sum(float v) {
+    if constexpr (LP == 8) {
+        v = sum_step<1>(v);
+        v = sum_step<2>(v);
+        return sum_step<4>(v);
+    } else {
+        v = row_sum16(v);
+        if constexpr (LP == 32) v = sum_step<16>(v);
+        return v;
+    }
 }
 
 // Per-head RMSNorm (optional) + RoPE of one head vector, one wave.  Writes the
@@ -793,28 +823,43 @@ __device__ __forceinline__ void rope_head(const float* src, const float* nw, flo
     }
 }
 
-// grid = (nkv, max_splits), 256 threads.  Block (h, s) covers positions
+// grid = (nkv, max_splits), 512 threads.  Block (h, s) covers positions
 // [s*chunk, min(L, (s+1)*chunk)) of KV head h for its G query heads.
+//
+// A launch this small is a chain of latencies, so a lane keeps one position
+// slot for scores, probabilities and P.V (HD/8 lanes a position, nothing goes
+// through LDS in between), each wave runs its own softmax over its slots, and
+// the waves are merged once: two barriers, and none of the block-wide maximum,
+// the score buffer or the 32-deep sums in LDS that took most of the time.  A
+// token through 8 layers and a small head: 8/4 heads of 64 at 100 positions 183
+// -> 153 us, 16/4 of 128 at 500 290 -> 265 and at 2000 349 -> 291, 8/2 of 256
+// at 500 371 -> 251 and at 2000 490 -> 274.
+template <int HD, int G> struct AttnShape {
+    static constexpr int LP = HD / 8;                 // lanes per position (16-byte chunks)
+    static constexpr int PPW = 64 / LP;               // positions per wave per tile
+    static constexpr int NW = 8;                      // waves
+    static constexpr int TILE = NW * PPW;             // positions per tile
+    // tiles per round, all requested at once (as many as the registers hold)
+    static constexpr int FIT = kAttnOne<HD> / TILE, CAP = G == 8 ? 2 : 8, PF = FIT < CAP ? FIT : CAP;
+};
 template <int HD, int G>
-__global__ __launch_bounds__(256) void k_attn_decode(AttnArgs a) {
-    constexpr int LP = HD / 8;          // lanes per position (16-byte chunks)
-    constexpr int PPW = 64 / LP;        // positions per wave per tile
-    constexpr int TILE = 4 * PPW;       // positions per tile
-    constexpr int PG = 256 / LP;        // position groups in P.V
+__global__ __launch_bounds__(512) void k_attn_decode(AttnArgs a) {
+    using S = AttnShape<HD, G>;
+    constexpr int LP = S::LP, PPW = S::PPW, NW = S::NW, TILE = S::TILE, PF = S::PF, NT = 64 * NW;
     constexpr int GD4 = G * HD / 4;     // float4 slices of the G output heads
-    constexpr int SG = 256 / GD4 > 0 ? 256 / GD4 : 1;   // split groups in the merge
-    extern __shared__ float smem[];
-    float* qs = smem;                   // [G][HD]
-    float* kn = qs + G * HD;            // [HD] newest K (fp16-rounded)
-    float* vn = kn + HD;                // [HD] newest V (fp16-rounded)
-    float* sc = vn + HD;                // [G][chunk_cap]
-    __shared__ float ml[2 * G];
+    constexpr int SG = NT / GD4 > 0 ? NT / GD4 : 1;   // split groups in the merge
+    constexpr int NV = 8 * G;           // P.V sums per lane
+    constexpr int RN = NW * G * HD > 6 * NT ? NW * G * HD : 6 * NT;
+    __shared__ float qs[G * HD];
+    __shared__ float kn[HD], vn[HD];    // newest K and V (fp16-rounded)
+    __shared__ float red[RN];           // [NW][G][HD]
+    __shared__ float wm[NW][G], wl[NW][G];
     __shared__ int is_last;
 
     const int pos = a.st->pos;
     const int L = pos + 1;
     int splits, chunk;
-    attn_plan(L, a.max_splits, splits, chunk);
+    attn_plan<HD>(L, a.max_splits, splits, chunk);
     const int s = blockIdx.y;
     if (s >= splits) return;
     const int kvh = blockIdx.x;
@@ -826,28 +871,31 @@ __global__ __launch_bounds__(256) void k_attn_decode(AttnArgs a) {
     const int nq = a.nkv * G, qd = nq * HD, kvd = a.nkv * HD;
     const int half = HD / 2;
     const float scale = 1.0f / sqrtf((float)HD);
-    const int sub = lane % LP, slot = lane / LP;
-    const int dsub = tid % LP, pg = tid / LP;
+    const int sub = lane % LP, slot0 = __builtin_amdgcn_readfirstlane(wave) * PPW, slot = slot0 + lane / LP;
 
-    // the first kAttnPf K tiles and V position groups: the cache loads are
-    // issued before anything else (the newest row, pos, comes from LDS)
-    uint4 kpre[kAttnPf], vpre[kAttnPf];
+    // a round's K and V rows, requested before anything else (the newest row,
+    // pos, comes from LDS)
+    uint4 kk[PF], vv[PF];
+    auto load = [&](int r0) __attribute__((always_inline)) {
 #pragma unroll
-    for (int t = 0; t < kAttnPf; t++) {
-        const int pik = t * TILE + wave * PPW + slot, piv = t * PG + pg;
-        kpre[t] = make_uint4(0, 0, 0, 0);
-        vpre[t] = make_uint4(0, 0, 0, 0);
-        if (pik < n && p0 + pik < pos)
-            kpre[t] = *reinterpret_cast<const uint4*>(a.kc + (size_t)(p0 + pik) * kvd + kvh * HD + sub * 8);
-        if (piv < n && p0 + piv < pos)
-            vpre[t] = *reinterpret_cast<const uint4*>(a.vc + (size_t)(p0 + piv) * kvd + kvh * HD + dsub * 8);
-    }
+        for (int t = 0; t < PF; t++) {
+            const int pi = r0 + t * TILE + slot;
+            kk[t] = make_uint4(0, 0, 0, 0);
+            vv[t] = make_uint4(0, 0, 0, 0);
+            if (pi < n && p0 + pi < pos) {
+                const size_t off = (size_t)(p0 + pi) * kvd + kvh * HD + sub * 8;
+                kk[t] = *reinterpret_cast<const uint4*>(a.kc + off);
+                vv[t] = *reinterpret_cast<const uint4*>(a.vc + off);
+            }
+        }
+    };
+    load(0);
 
     // QK-norm + RoPE of the G query heads (every block), and of the newest
     // K/V row (the block that holds position pos, which also appends it)
     const float* cr = a.cos_t + (size_t)pos * half;
     const float* sr = a.sin_t + (size_t)pos * half;
-    for (int t = wave; t < G + 2; t += 4) {
+    for (int t = wave; t < G + 2; t += NW) {
         if (t < G) {
             rope_head(a.qkv + (size_t)(kvh * G + t) * HD, a.q_norm, a.eps, cr, sr, HD, a.style,
                       qs + t * HD, nullptr, lane);
@@ -865,105 +913,134 @@ __global__ __launch_bounds__(256) void k_attn_decode(AttnArgs a) {
         }
     }
     __syncthreads();
-
-    // scores: tile t0 (positions t0 .. t0 + TILE - 1 of the split)
-    auto score_tile = [&](int t0, uint4 kv) {
-        const int pi = t0 + wave * PPW + slot;
-        const bool act = pi < n;
-        const int p = p0 + pi;
-        float kf[8];
-        if (act && p == pos) {
+    float qr[G][8];
 #pragma unroll
-            for (int e = 0; e < 8; e++) kf[e] = kn[sub * 8 + e];
-        } else {
-            const half2_t k01 = as_h2(kv.x), k23 = as_h2(kv.y), k45 = as_h2(kv.z), k67 = as_h2(kv.w);
-            kf[0] = (float)k01.x; kf[1] = (float)k01.y; kf[2] = (float)k23.x; kf[3] = (float)k23.y;
-            kf[4] = (float)k45.x; kf[5] = (float)k45.y; kf[6] = (float)k67.x; kf[7] = (float)k67.y;
+    for (int g = 0; g < G; g++)
+#pragma unroll
+        for (int e = 0; e < 8; e++) qr[g][e] = qs[g * HD + sub * 8 + e];
+
+    auto widen8 = [&](uint4 w, const float* newest, bool is_new, float (&f)[8]) __attribute__((always_inline)) {
+        const half2_t h0 = as_h2(w.x), h1 = as_h2(w.y), h2 = as_h2(w.z), h3 = as_h2(w.w);
+        f[0] = (float)h0.x; f[1] = (float)h0.y; f[2] = (float)h1.x; f[3] = (float)h1.y;
+        f[4] = (float)h2.x; f[5] = (float)h2.y; f[6] = (float)h3.x; f[7] = (float)h3.y;
+        if (is_new) {
+#pragma unroll
+            for (int e = 0; e < 8; e++) f[e] = newest[sub * 8 + e];
+        }
+    };
+    float m[G], l[G], acc[NV];
+#pragma unroll
+    for (int g = 0; g < G; g++) { m[g] = -INFINITY; l[g] = 0.0f; }
+#pragma unroll
+    for (int v = 0; v < NV; v++) acc[v] = 0.0f;
+    for (int r0 = 0; r0 < n; r0 += PF * TILE) {
+        if (r0 > 0) load(r0);
+        float sc[PF][G];
+#pragma unroll
+        for (int t = 0; t < PF; t++) {
+#pragma unroll
+            for (int g = 0; g < G; g++) sc[t][g] = -INFINITY;
+            if (r0 + t * TILE + slot0 >= n) continue;      // (the wave has no position there)
+            const int pi = r0 + t * TILE + slot;
+            float kf[8];
+            widen8(kk[t], kn, p0 + pi == pos, kf);
+#pragma unroll
+            for (int g = 0; g < G; g++) {
+                float pd = qr[g][0] * kf[0];
+#pragma unroll
+                for (int e = 1; e < 8; e++) pd = pd + qr[g][e] * kf[e];
+                pd = pos_sum<LP>(pd) * scale;
+                sc[t][g] = pi < n ? pd : -INFINITY;
+            }
         }
 #pragma unroll
         for (int g = 0; g < G; g++) {
-            const float* qq = qs + g * HD + sub * 8;
-            float pd = qq[0] * kf[0];
+            float mx = sc[0][g];
 #pragma unroll
-            for (int e = 1; e < 8; e++) pd = pd + qq[e] * kf[e];
-            if constexpr (LP == 16) pd = row_sum16(pd);   // DPP within the 16-lane row
-            else pd = group_sum(pd, LP);
-            if (act && sub == 0) sc[g * a.chunk_cap + pi] = pd * scale;
+            for (int t = 1; t < PF; t++) mx = fmaxf(mx, sc[t][g]);
+            mx = max_step<32>(mx);
+            if constexpr (LP <= 16) mx = max_step<16>(mx);
+            if constexpr (LP <= 8) mx = max_step<8>(mx);
+            const float mn = fmaxf(m[g], mx);
+            const float ref = mn == -INFINITY ? 0.0f : mn;   // no score above -inf yet: p = 0
+            const float alpha = expf(m[g] - ref);
+            m[g] = mn;
+            l[g] = l[g] * alpha;
+#pragma unroll
+            for (int e = 0; e < 8; e++) acc[8 * g + e] = acc[8 * g + e] * alpha;
+#pragma unroll
+            for (int t = 0; t < PF; t++) {
+                sc[t][g] = expf(sc[t][g] - ref);
+                l[g] += sc[t][g];
+            }
         }
-    };
 #pragma unroll
-    for (int t = 0; t < kAttnPf; t++)
-        if (t * TILE < n) score_tile(t * TILE, kpre[t]);
-    for (int t0 = kAttnPf * TILE; t0 < n; t0 += TILE) {
-        const int pi = t0 + wave * PPW + slot;
-        uint4 kv = make_uint4(0, 0, 0, 0);
-        if (pi < n && p0 + pi < pos) kv = *reinterpret_cast<const uint4*>(a.kc + (size_t)(p0 + pi) * kvd + kvh * HD + sub * 8);
-        score_tile(t0, kv);
+        for (int t = 0; t < PF; t++) {
+            if (r0 + t * TILE + slot0 >= n) continue;
+            const int pi = r0 + t * TILE + slot;
+            float vf[8];
+            widen8(vv[t], vn, p0 + pi == pos, vf);
+#pragma unroll
+            for (int g = 0; g < G; g++)
+#pragma unroll
+                for (int e = 0; e < 8; e++) acc[8 * g + e] = acc[8 * g + e] + vf[e] * sc[t][g];
+        }
     }
-    __syncthreads();
-
-    for (int g = wave; g < G; g += 4) {
-        float m = -1e30f;
-        for (int i = lane; i < n; i += 64) m = fmaxf(m, sc[g * a.chunk_cap + i]);
-        m = wave_max_dpp(m);
-        float l = 0.0f;
-        for (int i = lane; i < n; i += 64) {
-            const float e = expf(sc[g * a.chunk_cap + i] - m);
-            sc[g * a.chunk_cap + i] = e;
-            l += e;
-        }
-        l = wave_sum_dpp(l);
+    // over the wave's position slots: the sums are scattered, a lane ends with
+    // NV / PPW of them starting at v0
+    int v0 = 0, nv = NV;
+    rs_step<32, NV>(acc, nv, lane);
+    nv /= 2;
+    v0 += (lane & 32) ? nv : 0;
+    if constexpr (LP <= 16) {
+        rs_step<16, NV>(acc, nv, lane);
+        nv /= 2;
+        v0 += (lane & 16) ? nv : 0;
+    }
+    if constexpr (LP <= 8) {
+        rs_step<8, NV>(acc, nv, lane);
+        nv /= 2;
+        v0 += (lane & 8) ? nv : 0;
+    }
+#pragma unroll
+    for (int v = 0; v < NV / PPW; v++) {
+        const int i = v0 + v;
+        red[(wave * G + i / 8) * HD + sub * 8 + i % 8] = acc[v];
+    }
+#pragma unroll
+    for (int g = 0; g < G; g++) {
+        float t = sum_step<32>(l[g]);
+        if constexpr (LP <= 16) t = sum_step<16>(t);
+        if constexpr (LP <= 8) t = sum_step<8>(t);
         if (lane == 0) {
-            ml[2 * g] = m;
-            ml[2 * g + 1] = l;
+            wm[wave][g] = m[g];
+            wl[wave][g] = t;
         }
     }
     __syncthreads();
-
-    // P.V: thread = (position group, 8-wide slice of the head dimension)
-    float acc[G][8];
+    // the waves' weights and the split's maximum and sum for head g
+    auto wave_weights = [&](int g, float (&f)[NW], float& ms, float& lsum) __attribute__((always_inline)) {
+        ms = wm[0][g];
 #pragma unroll
-    for (int g = 0; g < G; g++)
+        for (int w = 1; w < NW; w++) ms = fmaxf(ms, wm[w][g]);
+        const float ref = ms == -INFINITY ? 0.0f : ms;
+        lsum = 0.0f;
 #pragma unroll
-        for (int e = 0; e < 8; e++) acc[g][e] = 0.0f;
-    auto pv_row = [&](int pi, uint4 vv) {
-        const int p = p0 + pi;
-        float vf[8];
-        if (p == pos) {
-#pragma unroll
-            for (int e = 0; e < 8; e++) vf[e] = vn[dsub * 8 + e];
-        } else {
-            const half2_t v01 = as_h2(vv.x), v23 = as_h2(vv.y), v45 = as_h2(vv.z), v67 = as_h2(vv.w);
-            vf[0] = (float)v01.x; vf[1] = (float)v01.y; vf[2] = (float)v23.x; vf[3] = (float)v23.y;
-            vf[4] = (float)v45.x; vf[5] = (float)v45.y; vf[6] = (float)v67.x; vf[7] = (float)v67.y;
-        }
-#pragma unroll
-        for (int g = 0; g < G; g++) {
-            const float pw = sc[g * a.chunk_cap + pi];
-#pragma unroll
-            for (int e = 0; e < 8; e++) acc[g][e] = acc[g][e] + vf[e] * pw;
+        for (int w = 0; w < NW; w++) {
+            f[w] = expf(wm[w][g] - ref);
+            lsum = lsum + wl[w][g] * f[w];
         }
     };
-#pragma unroll
-    for (int t = 0; t < kAttnPf; t++)
-        if (t * PG + pg < n) pv_row(t * PG + pg, vpre[t]);
-    for (int pi = kAttnPf * PG + pg; pi < n; pi += PG)
-        pv_row(pi, *reinterpret_cast<const uint4*>(a.vc + (size_t)(p0 + pi) * kvd + kvh * HD + dsub * 8));
-    __syncthreads();   // scores no longer needed: smem is reused for the cross-group sum
-    float* red = smem; // [PG][G][HD]
-#pragma unroll
-    for (int g = 0; g < G; g++)
-#pragma unroll
-        for (int e = 0; e < 8; e++) red[(pg * G + g) * HD + dsub * 8 + e] = acc[g][e];
-    __syncthreads();
     if (splits == 1) {
         // the only split: its sums are final (the merge of one record
         // computes the same quotient), so no record, arrival or merge
-        for (int i = tid; i < G * HD; i += 256) {
-            const int g = i / HD, d = i % HD;
-            float sum = 0.0f;
-            for (int k = 0; k < PG; k++) sum += red[(k * G + g) * HD + d];
-            a.out16[(size_t)(kvh * G + g) * HD + d] = f32_to_f16_bits(sum / ml[2 * g + 1]);
+        for (int i = tid; i < G * HD; i += NT) {
+            const int g = i / HD;
+            float f[NW], ms, ls, sum = 0.0f;
+            wave_weights(g, f, ms, ls);
+#pragma unroll
+            for (int w = 0; w < NW; w++) sum = sum + red[w * G * HD + i] * f[w];
+            a.out16[(size_t)kvh * G * HD + i] = f32_to_f16_bits(sum / ls);
         }
         return;
     }
@@ -977,20 +1054,23 @@ __global__ __launch_bounds__(256) void k_attn_decode(AttnArgs a) {
     constexpr int RH = HD + 4;              // floats per head in a record
     const auto prs = __builtin_amdgcn_make_buffer_rsrc(a.part, (short)0, 0x7fffffff, 0x00020000);
     const unsigned rec0 = (unsigned)(((size_t)kvh * a.max_splits + s) * G * RH * 4);
-    for (int i4 = tid; i4 < G * HD / 4; i4 += 256) {
+    for (int i4 = tid; i4 < GD4; i4 += NT) {
         const int g = (4 * i4) / HD, d = (4 * i4) % HD;
+        float f[NW], ms, ls;
+        wave_weights(g, f, ms, ls);
         float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
-        for (int k = 0; k < PG; k++) {
-            const float4 r = *reinterpret_cast<const float4*>(red + (k * G + g) * HD + d);
-            sum.x += r.x; sum.y += r.y; sum.z += r.z; sum.w += r.w;
+#pragma unroll
+        for (int w = 0; w < NW; w++) {
+            const float4 r = *reinterpret_cast<const float4*>(red + (w * G + g) * HD + d);
+            sum.x += r.x * f[w]; sum.y += r.y * f[w]; sum.z += r.z * f[w]; sum.w += r.w * f[w];
         }
         __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, sum), prs,
                                                rec0 + (unsigned)(g * RH + d) * 4, 0, 16);
-    }
-    if (tid < G) {
-        const float4 t4 = make_float4(ml[2 * tid], ml[2 * tid + 1], 0.f, 0.f);
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, t4), prs,
-                                               rec0 + (unsigned)(tid * RH + HD) * 4, 0, 16);
+        if (d == 0) {
+            const float4 t4 = make_float4(ms, ls, 0.f, 0.f);
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, t4), prs,
+                                                   rec0 + (unsigned)(g * RH + HD) * 4, 0, 16);
+        }
     }
 
     // the last block of this KV head merges all splits
@@ -1003,7 +1083,7 @@ __global__ __launch_bounds__(256) void k_attn_decode(AttnArgs a) {
     if (!is_last) return;
     const unsigned base = (unsigned)((size_t)kvh * a.max_splits * G * RH * 4);
     const unsigned stride = (unsigned)(G * RH * 4);
-    float m = -INFINITY, l = 0.0f, o[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    float mm = -INFINITY, lm = 0.0f, o[4] = {0.0f, 0.0f, 0.0f, 0.0f};
     const int gd = tid % GD4, sg = tid / GD4;
     const int g = gd / (HD / 4), d4 = (gd % (HD / 4)) * 4;
     if (sg < SG) {
@@ -1023,22 +1103,22 @@ __global__ __launch_bounds__(256) void k_attn_decode(AttnArgs a) {
             for (int j = 0; j < kMergeB; j++) {
                 if (sp0 + j * SG >= splits) break;
                 const float msj = __uint_as_float(ml4[j].x), lsj = __uint_as_float(ml4[j].y);
-                const float mn = fmaxf(m, msj);
-                const float fa = expf(m - mn), fb = expf(msj - mn);
-                l = l * fa + lsj * fb;
+                const float mn = fmaxf(mm, msj), ref = mn == -INFINITY ? 0.0f : mn;
+                const float fa = expf(mm - ref), fb = expf(msj - ref);
+                lm = lm * fa + lsj * fb;
                 o[0] = o[0] * fa + __uint_as_float(os4[j].x) * fb;
                 o[1] = o[1] * fa + __uint_as_float(os4[j].y) * fb;
                 o[2] = o[2] * fa + __uint_as_float(os4[j].z) * fb;
                 o[3] = o[3] * fa + __uint_as_float(os4[j].w) * fb;
-                m = mn;
+                mm = mn;
             }
         }
     }
     __syncthreads();
-    float* mr = smem;                       // [SG][GD4][6]
+    float* mr = red;                        // [SG][GD4][6]
     if (sg < SG) {
         float* r = mr + (sg * GD4 + gd) * 6;
-        r[0] = m; r[1] = l; r[2] = o[0]; r[3] = o[1]; r[4] = o[2]; r[5] = o[3];
+        r[0] = mm; r[1] = lm; r[2] = o[0]; r[3] = o[1]; r[4] = o[2]; r[5] = o[3];
     }
     __syncthreads();
     if (sg == 0) {
@@ -1171,8 +1251,8 @@ int mdx_launch_advance(mdx_state* state, int advance, void* stream) {
 }
 
 int mdx_attn_max_splits(int max_seq) {
-    (void)max_seq;
-    return 64;
+    const int s = (max_seq + kAttnChunk - 1) / kAttnChunk;
+    return s < 1 ? 1 : (s > 64 ? 64 : s);
 }
 
 size_t mdx_attn_decode_scratch_bytes(int nq, int nkv, int hd, int max_splits) {
@@ -1199,23 +1279,13 @@ int mdx_launch_attn_decode(const mdx_state* state, const float* qkv, const float
     a.vc = v_cache;
     a.nkv = nkv;
     a.max_splits = max_splits;
-    a.chunk_cap = (max_seq + max_splits - 1) / max_splits;
-    if (a.chunk_cap < kAttnChunk) a.chunk_cap = kAttnChunk;
     a.part = (float*)scratch;
     a.done = (unsigned int*)((char*)scratch + (size_t)nq * max_splits * (hd + 4) * 4);
     a.out16 = attn_out16;
-    const int LP = hd / 8;
-    const int PG = 256 / LP;
-    const size_t lds_a = (size_t)(G * hd + 2 * hd + G * a.chunk_cap) * 4;
-    const size_t lds_b = (size_t)PG * G * hd * 4;
-    const size_t lds_c = (size_t)256 * 6 * 4;
-    size_t lds = lds_a > lds_b ? lds_a : lds_b;
-    if (lds_c > lds) lds = lds_c;
-    if (lds > 64 * 1024) return -5;
     dim3 grid(nkv, max_splits);
 #define MDX_ATTN(HD_, G_)                                                                          \
     if (hd == HD_ && G == G_) {                                                                    \
-        hipLaunchKernelGGL((k_attn_decode<HD_, G_>), grid, dim3(256), lds, (hipStream_t)stream, a); \
+        hipLaunchKernelGGL((k_attn_decode<HD_, G_>), grid, dim3(512), 0, (hipStream_t)stream, a); \
         return hipGetLastError() == hipSuccess ? 0 : -4;                                           \
     }
     MDX_ATTN(64, 1) MDX_ATTN(64, 2) MDX_ATTN(64, 4) MDX_ATTN(64, 8)
