@@ -59,7 +59,7 @@ struct MatmulDecoderContext {
     void* d_sscr;                /* sampler scratch */
     void* d_part;            /* attention split partials + merge counters */
     uint16_t *d_attn16, *d_act16;
-    void* d_partial;         /* lm_head argmax key + completion counter */
+    void* d_partial;         /* lm_head argmax keys and arrival counters */
     int* d_tokens;
     int tokens_cap;
     float *d_bhidden, *d_bqkv, *d_bq, *d_gscr;
