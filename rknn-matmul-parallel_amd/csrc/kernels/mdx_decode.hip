@@ -948,7 +948,7 @@ __global__ __launch_bounds__(512) void k_attn_decode(AttnArgs a) {
             for (int g = 0; g < G; g++) {
                 float pd = qr[g][0] * kf[0];
 #pragma unroll
-                for (int e = 1; e < 8; e++) pd = pd + qr[g][e] * kf[e];
+                for (int e = 1; e < 8; e++) pd = fmaf(qr[g][e], kf[e], pd);
                 pd = pos_sum<LP>(pd) * scale;
                 sc[t][g] = pi < n ? pd : -INFINITY;
             }
@@ -983,7 +983,7 @@ __global__ __launch_bounds__(512) void k_attn_decode(AttnArgs a) {
 #pragma unroll
             for (int g = 0; g < G; g++)
 #pragma unroll
-                for (int e = 0; e < 8; e++) acc[8 * g + e] = acc[8 * g + e] + vf[e] * sc[t][g];
+                for (int e = 0; e < 8; e++) acc[8 * g + e] = fmaf(vf[e], sc[t][g], acc[8 * g + e]);
         }
     }
     // over the wave's position slots: the sums are scattered, a lane ends with
