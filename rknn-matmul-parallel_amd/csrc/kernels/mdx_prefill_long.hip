@@ -24,7 +24,6 @@ namespace {
 typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
 
 constexpr int kKT = 64;            // k per LDS stage
-constexpr int kRun = 4;            // stages per partial sum
 constexpr int kStageChunks = kKT / 8;   // 16-byte chunks per LDS row
 
 // Where a tile's 16-byte chunk of row r goes: chunks are permuted within the
@@ -50,6 +49,7 @@ struct LongArgs {
     const float* scale;       // [N] or NULL
     int M, K, N;
     int tiles_m, tiles_n, splits, per_split;   // per_split: LDS stages per split
+    int run;                  // stages per partial sum
     float* out;               // LE_STORE [M][N]; LE_PART [splits][M][N], unscaled
     uint16_t* out16;          // LE_SWIGLU [M][N/2]
     // LE_ROPE
@@ -251,9 +251,7 @@ __global__ __launch_bounds__(256, 2) void k_long_gemm(LongArgs a) {
         }
     };
 
-    // sums of kRun stages (256 k) are added to a second set: one running sum
-    // over all of K loses precision (K = 3072: 3.5e-7 off the exact products'
-    // sum in the 2-norm, against 1.2e-7 so)
+    // sums of a.run stages (long_run) are added to a second set
     float4_t acc[NT][MT], tot[NT][MT];
 #pragma unroll
     for (int t = 0; t < NT; t++)
@@ -265,6 +263,7 @@ __global__ __launch_bounds__(256, 2) void k_long_gemm(LongArgs a) {
     stash(0, 0, s0);
     load(0, s0 + PD);
     __syncthreads();
+    int left = a.run;
     for (int sb = s0; sb < s1; sb += PD) {
 #pragma unroll
         for (int d = 0; d < PD; d++) {
@@ -290,7 +289,8 @@ __global__ __launch_bounds__(256, 2) void k_long_gemm(LongArgs a) {
                         acc[t][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wa, xb[j], acc[t][j], 0, 0, 0);
                 }
             }
-            if ((st - s0) % kRun == kRun - 1) {
+            if (--left == 0) {
+                left = a.run;
 #pragma unroll
                 for (int t = 0; t < NT; t++)
 #pragma unroll
@@ -384,8 +384,18 @@ __global__ __launch_bounds__(256, 2) void k_long_gemm(LongArgs a) {
 // of that product is the order in which a lane holds its scores).
 //
 // Queries and probabilities are fp32: each goes in as the sum of two fp16
-// values (22 bits), the queries scaled per row so that neither part leaves the
-// fp16 range, the probabilities by 2^6 relative to a reference score.
+// values, both rounded to nearest (23 bits), the queries scaled per row so that
+// neither part leaves the fp16 range, the probabilities by 2^6.  What this must
+// not lose against fp32 arithmetic (k_attn_prefill) is kept by the order of the
+// sums: a product's second parts go first, the scores are summed over 64
+// dimensions at a time (32 at 64 dimensions), the tile's P.V is summed from
+// zero and then added, and the exponent's offset is the reference score alone
+// (an offset of 6 more rounds every exponent at 2^-22).  Outputs rounded
+// otherwise than the exact result rounds, per thousand, before these / now /
+// k_attn_prefill, normal inputs, 16 heads of 128 over 8: M = 515 1.87 / 0.98 /
+// 1.03, M = 2000 2.11 / 1.11 / 1.16, equal scores 1.13 / 0.49 / 0.62; 8 of 256
+// over 2, M = 515: 2.10 / 0.98 / 0.98.  Their cost at M = 2000: 69.3 -> 70.2
+// us; 256 dimensions 159 -> 135 us (independent sums).
 //
 // The vector unit is what bounds it (at M = 2000 the longest block's tile took
 // 2.9 us with expf and a rescale per tile): the exponentials are v_exp_f32 of
@@ -410,21 +420,12 @@ __device__ __forceinline__ uint32_t max_exp(uint32_t m, u32x4_t v) {
 }
 __device__ __forceinline__ bool exp_nonfinite(uint32_t m) { return (m & 0xffffu) >= 0x7c00u || (m >> 16) >= 0x7c00u; }
 
-// fp32 pairs as the sums of two fp16 values: the first part rounds towards
-// zero (one instruction for both), the second holds the remainder.
-__device__ __forceinline__ void split16(float a, float b, half2_t& hi, half2_t& lo) {
-    hi = __builtin_bit_cast(half2_t, __builtin_amdgcn_cvt_pkrtz(a, b));
-    lo = half2_t{(_Float16)(a - (float)hi.x), (_Float16)(b - (float)hi.y)};
-}
+// fp32 values as the sums of two fp16 values.
 __device__ __forceinline__ void split16(const float (&v)[8], half8_t& hi, half8_t& lo) {
 #pragma unroll
-    for (int e = 0; e < 8; e += 2) {
-        half2_t h, l;
-        split16(v[e], v[e + 1], h, l);
-        hi[e] = h.x;
-        hi[e + 1] = h.y;
-        lo[e] = l.x;
-        lo[e + 1] = l.y;
+    for (int e = 0; e < 8; e++) {
+        hi[e] = (_Float16)v[e];
+        lo[e] = (_Float16)(v[e] - (float)hi[e]);
     }
 }
 
@@ -436,6 +437,7 @@ __global__ __launch_bounds__(512, 2) void k_attn_long(int pos0, int M, const flo
     constexpr int TB = 64 / G;             // positions per block
     constexpr int KB = HD == 256 ? 32 : 64;   // keys per tile (32: no spills at 256 dimensions)
     constexpr int DS = HD / 32;            // k-steps of a score
+    constexpr int NS = HD == 256 ? 4 : 2;  // sums of a score
     constexpr int DT = HD / 16;            // 16-row tiles of O^T
     constexpr int KS = HD / 8 + 1;         // uint4 per LDS row of K (16-byte pad)
     constexpr int VS = KB / 8 + 1;         // uint4 per LDS row of V^T
@@ -557,7 +559,7 @@ __global__ __launch_bounds__(512, 2) void k_attn_long(int pos0, int M, const flo
         load(p0 + 2 * KB);
 
         // scores: s[kt][i] = key p0 + 16 kt + 4 g + i, then 2^6 times their
-        // exponentials relative to the reference
+        // exponentials relative to the reference (ls: the sum of these, unscaled)
         float4_t s[KB / 16];
         float ls, next;
         auto softmax = [&]() __attribute__((always_inline)) {
@@ -574,7 +576,7 @@ __global__ __launch_bounds__(512, 2) void k_attn_long(int pos0, int M, const flo
                 mx = fmaxf(mx, fmaxf(fmaxf(s[kt][0], s[kt][1]), fmaxf(s[kt][2], s[kt][3])));
             const float m2 = rows_max4(mx) * c;
             next = m2 > ref + 8.0f ? m2 : ref;          // (the first score: ref is -inf)
-            const float off = next == -INFINITY ? 0.0f : 6.0f - next;
+            const float off = next == -INFINITY ? 0.0f : -next;
             ls = 0.0f;
 #pragma unroll
             for (int kt = 0; kt < KB / 16; kt++)
@@ -582,17 +584,28 @@ __global__ __launch_bounds__(512, 2) void k_attn_long(int pos0, int M, const flo
                 for (int i = 0; i < 4; i++) {
                     s[kt][i] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[kt][i], c, off));
                     ls = ls + s[kt][i];
+                    s[kt][i] = s[kt][i] * 64.0f;
                 }
         };
 #pragma unroll
         for (int kt = 0; kt < KB / 16; kt++) {
-            s[kt] = float4_t{0.f, 0.f, 0.f, 0.f};
+            float4_t sum[NS];
+            half8_t k8[DS];
+#pragma unroll
+            for (int n = 0; n < NS; n++) sum[n] = float4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int d = 0; d < DS; d++) {
-                const half8_t k8 = __builtin_bit_cast(half8_t, ks[(16 * kt + c16) * KS + 4 * d + g]);
-                s[kt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(k8, qh[d], s[kt], 0, 0, 0);
-                s[kt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(k8, ql[d], s[kt], 0, 0, 0);
+                k8[d] = __builtin_bit_cast(half8_t, ks[(16 * kt + c16) * KS + 4 * d + g]);
+                sum[0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(k8[d], ql[d], sum[0], 0, 0, 0);
             }
+#pragma unroll
+            for (int d = 0; d < DS; d++)
+                sum[d * NS / DS] = __builtin_amdgcn_mfma_f32_16x16x32_f16(k8[d], qh[d], sum[d * NS / DS], 0, 0, 0);
+#pragma unroll
+            for (int n = 1; n < NS; n *= 2)
+#pragma unroll
+                for (int e = 0; e < NS; e += 2 * n) sum[e] += sum[e + n];
+            s[kt] = sum[0];
         }
         softmax();
         if (__any(ls != ls)) {
@@ -620,18 +633,26 @@ __global__ __launch_bounds__(512, 2) void k_attn_long(int pos0, int M, const flo
         }
         runL = runL + ls;
         if (!slow) {
+            half8_t ph[KB / 32], pl[KB / 32];
 #pragma unroll
             for (int pr = 0; pr < KB / 32; pr++) {
                 const float pv[8] = {s[2 * pr][0], s[2 * pr][1], s[2 * pr][2], s[2 * pr][3],
                                      s[2 * pr + 1][0], s[2 * pr + 1][1], s[2 * pr + 1][2], s[2 * pr + 1][3]};
-                half8_t ph, pl;
-                split16(pv, ph, pl);
+                split16(pv, ph[pr], pl[pr]);
+            }
 #pragma unroll
-                for (int d = 0; d < DT; d++) {
-                    const half8_t v8 = __builtin_bit_cast(half8_t, vs[(16 * d + c16) * VS + 4 * pr + g]);
-                    o[d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(v8, ph, o[d], 0, 0, 0);
-                    o[d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(v8, pl, o[d], 0, 0, 0);
+            for (int d = 0; d < DT; d++) {
+                float4_t t = float4_t{0.f, 0.f, 0.f, 0.f};
+                half8_t v8[KB / 32];
+#pragma unroll
+                for (int pr = 0; pr < KB / 32; pr++) {
+                    v8[pr] = __builtin_bit_cast(half8_t, vs[(16 * d + c16) * VS + 4 * pr + g]);
+                    t = __builtin_amdgcn_mfma_f32_16x16x32_f16(v8[pr], pl[pr], t, 0, 0, 0);
                 }
+#pragma unroll
+                for (int pr = 0; pr < KB / 32; pr++)
+                    t = __builtin_amdgcn_mfma_f32_16x16x32_f16(v8[pr], ph[pr], t, 0, 0, 0);
+                o[d] += t;
             }
         } else {
             __syncthreads();                // every wave is done with the K tile
@@ -676,7 +697,7 @@ __global__ __launch_bounds__(512, 2) void k_attn_long(int pos0, int M, const flo
     for (int d = 0; d < DT; d++)
 #pragma unroll
         for (int i = 0; i < 4; i++) o[d][i] = o[d][i] * a0 + mg[(4 * d + i) * 256] * a1;
-    const float l = rows_sum4(runL * a0 + mg[(4 * DT + 1) * 256] * a1);
+    const float l = 64.0f * rows_sum4(runL * a0 + mg[(4 * DT + 1) * 256] * a1);
     uint16_t* dst = out16 + ((size_t)t * nq + hq) * HD + 4 * g;
 #pragma unroll
     for (int d = 0; d < DT; d++) {
@@ -716,6 +737,22 @@ LongTile long_tile(int M, int N, int K, bool can_split, bool wide) {
     return t;
 }
 
+// Stages per partial sum.  A chain of sums rounds at the size it has reached,
+// so few long ones and many short ones both lose, and products of 4-bit
+// weights, short enough to be summed almost exactly inside an MFMA, want the
+// longest.  Off the exact sums by (2-norm, 1e-8) at 1 / 2 / 4 stages, and the
+// eight interleaved sums of the 64-row kernels, which these must not exceed:
+// fp16 K = 256 7.0 / 8.0 / 10.4, 7.1; 576 8.2 / 8.8 / -, 8.4; 1024 9.6 / 9.5 /
+// 11.2, 9.5; 3072 14.0 / 12.0 / 12.5, 13.9; 4096 - / 13.1 / 13.0, 15.7; int8 K
+// = 512 7.4 / 7.5 / 9.3, 7.4; 1024 9.1 / 8.4 / 9.7, 8.4; 4096 - / 12.4 / 11.8,
+// 14.0; int4, at 2 / 4 / this rule: K = 1536 7.2 / 6.5 / 6.5, 6.5; 4096 11.0 /
+// 8.9 / 8.2, 8.2.  One chain over 3072 of fp16: 35.  The additions do not show
+// in the time (fp16 2000 x 1024 x 6144 at 1 / 2 / 4: 52.4 / 55.2 / 54.3 us).
+int long_run(int kind, int stages) {
+    if (kind == MDX_W_I4) return 2 * cdiv(stages, 16);
+    return stages <= (kind == MDX_W_F16 ? 12 : 8) ? 1 : (stages <= 48 ? 2 : 4);
+}
+
 template <int KIND, int EPI, int HD>
 int long_launch_kind(const LongArgs& a, const LongTile& t, hipStream_t s) {
     dim3 grid((unsigned)(a.tiles_m * a.tiles_n * a.splits)), block(256);
@@ -735,6 +772,7 @@ int long_launch(LongArgs& a, int kind, const LongTile& t, void* stream) {
     a.tiles_n = EPI == LE_SWIGLU ? cdiv(a.N / 2, t.bn / 2) : cdiv(a.N, t.bn);
     a.splits = t.splits;
     a.per_split = cdiv(cdiv(a.K, kKT), t.splits);
+    a.run = long_run(kind, a.per_split);
     if ((long long)a.tiles_m * a.tiles_n * a.splits > 0x7fffffffLL) return -1;
     hipStream_t s = (hipStream_t)stream;
     switch (kind) {
