@@ -1122,13 +1122,16 @@ __global__ __launch_bounds__(512) void k_attn_decode(AttnArgs a) {
     }
     __syncthreads();
     if (sg == 0) {
+        // the groups that hold records; one of maximum -inf counts too, its sums
+        // are NaN when its scores (or a value of probability 0) were
+        const int ng = min(SG, splits);
         float M = -INFINITY;
-        for (int k = 0; k < SG; k++) M = fmaxf(M, mr[(k * GD4 + gd) * 6]);
+        for (int k = 0; k < ng; k++) M = fmaxf(M, mr[(k * GD4 + gd) * 6]);
+        const float ref = M == -INFINITY ? 0.0f : M;
         float Ls = 0.0f, O[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-        for (int k = 0; k < SG; k++) {
+        for (int k = 0; k < ng; k++) {
             const float* r = mr + (k * GD4 + gd) * 6;
-            if (r[0] == -INFINITY) continue;
-            const float f = expf(r[0] - M);
+            const float f = expf(r[0] - ref);
             Ls = Ls + r[1] * f;
             for (int e = 0; e < 4; e++) O[e] = O[e] + r[2 + e] * f;
         }
