@@ -201,7 +201,8 @@ __global__ __launch_bounds__(256, 2) void k_long_gemm(LongArgs a) {
     // load under a branch makes it wait for all: M = 203, K = 1024 took 1 us a
     // stage whatever PD).  Rows past the edge repeat the last row (their
     // results are not stored), stages past the last repeat it, and k past K
-    // repeat the row's last load and become zeros on their way to LDS.
+    // repeat the row's last load and become zeros on their way to LDS, in both
+    // operands: a repeated weight may be an infinity (fp16 ones only).
     const uint16_t* xp[XU];
     int xk[XU], xl[XU];
 #pragma unroll
@@ -237,6 +238,11 @@ __global__ __launch_bounds__(256, 2) void k_long_gemm(LongArgs a) {
 #pragma unroll
             for (int i = 0; i < XU; i++)
                 if (st * kKT + xk[i] >= a.K) xv[d][i] = u32x4_t{0u, 0u, 0u, 0u};
+            if constexpr (KIND == MDX_W_F16) {
+#pragma unroll
+                for (int i = 0; i < WU; i++)
+                    if (st * kKT + wk[i] >= a.K) wv[d][i] = u32x4_t{0u, 0u, 0u, 0u};
+            }
         }
 #pragma unroll
         for (int i = 0; i < XU; i++) xs[buf][xl[i]] = __builtin_bit_cast(uint4, xv[d][i]);

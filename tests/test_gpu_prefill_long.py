@@ -77,6 +77,27 @@ def test_long_projections_as_exact_as_64_row_ones(mdx, gpu, kind, K):
         np.concatenate([mdx.gemm_residual(kind, 64, K, N, w, s, x[r], h0[r], None)[0] for r in halves]))
 
 
+@pytest.mark.parametrize("M,K,N", [(70, 32, 64), (100, 96, 64), (65, 352, 128), (203, 1056, 1024), (130, 128, 64)])
+def test_long_gemm_infinite_weights(mdx, gpu, M, K, N):
+    """Infinite fp16 weights, also among the last k of a K that ends inside a
+    stage of 64, give infinities (of both signs in one column: NaN)."""
+    rng = np.random.default_rng(K)
+    x = rng.uniform(0.5, 1.5, (M, K)).astype(np.float16).astype(np.float32)
+    w = (rng.standard_normal((K, N)) * 0.02).astype(np.float16)
+    w[K - 1, 3], w[K - 8, 5], w[0, 7], w[K - 1, 9] = np.inf, -np.inf, np.inf, np.nan
+    w[K - 2, 11], w[K - 3, 11] = np.inf, -np.inf
+    with np.errstate(invalid="ignore"):
+        ref = x.astype(np.float64) @ w.astype(np.float64)
+    h0 = rng.standard_normal((M, N)).astype(np.float32)
+    wu = w.view(np.uint16)
+    for y, r in ((mdx.gemm(0, M, K, N, wu, None, x, long=True), ref),
+                 (mdx.gemm_residual(0, M, K, N, wu, None, x, h0, None, long=True)[0], h0 + ref)):
+        assert np.array_equal(np.isnan(y), np.isnan(r)) and np.array_equal(np.isinf(y), np.isinf(r))
+        assert np.array_equal(np.sign(y[np.isinf(r)]), np.sign(r[np.isinf(r)]))
+        ok = np.isfinite(r)
+        assert rel_err(y[ok], r[ok]) < GEMM_TOL
+
+
 def _attention64(q, k, v, S, M, nq, nkv, hd):
     out = np.empty((M, nq, hd))
     for h in range(nq):
