@@ -1567,7 +1567,10 @@ int mdx_prefill_logits(MatmulDecoderContext* c, const float* embeddings, int M, 
     if (!rc) rc = run_head(c, &c->lm, c->h_io, NULL, 0, c->h_res, c->stream);
     if (!rc) rc = mdxrt_signal(&c->h_res->done, NULL, c->stream);
     if (!rc) rc = mdxrt_wait(&c->h_res->done, c->stream);
-    if (rc) return MATMUL_DECODER_ERR_RKNN;
+    if (rc) {   /* a head already issued writes h_io and h_res */
+        mdxrt_stream_sync(c->stream);
+        return MATMUL_DECODER_ERR_RKNN;
+    }
     if (logits) memcpy(logits, c->h_io, (size_t)c->V * 4);
     return c->h_res->argmax;
 }
