@@ -1284,17 +1284,18 @@ static int run_step(MatmulDecoderContext* c, int token_id, const float* embeddin
     if (!count) return tok;
     const float total = (float)(md_now_ms() - t0);
     /* Device times from the kernels: layers_ms is the layers' (with the lm_head
-     * too when it runs inside the one launch), head_ms the rest.  Without
+     * too when it runs inside the one launch), head_ms the lm_head kernel's.
+     * The copies and the draw behind it count as convert_ms.  Without
      * MDX_PROFILE the one launch is not split: it all counts as matmul_ms. */
     const mdx_host_res* r = c->h_res;
     const unsigned long long mid = r->t_layers ? r->t_layers : r->t_end;
     const float layers_ms = (float)(mid - r->t_start) * c->clock_ms;
-    const float head_ms = (float)(r->t_end - mid) * c->clock_ms;
+    const float head_ms = lm && !one ? (float)(r->t_head - mid) * c->clock_ms : 0.0f;
     c->stats.total_ms = total;
     c->stats.matmul_ms = layers_ms;
     c->stats.rebind_ms = 0.0f;
     c->stats.cpu_ops_ms = 0.0f;
-    c->stats.lm_head_ms = lm && !one ? head_ms : 0.0f;
+    c->stats.lm_head_ms = head_ms;
     if (prof) {
         profile_split(c, layers_ms, one, &c->stats);
         if (lm && !one) c->stats.lm_head_ms = head_ms;

@@ -394,6 +394,7 @@ __device__ __forceinline__ void lm_finish(const GemvArgs& a, unsigned long long 
         if (a.res) {
             a.res->argmax = tok;
             a.res->t_layers = t_begin;
+            a.res->t_head = wall_clock64();
         }
     }
 }

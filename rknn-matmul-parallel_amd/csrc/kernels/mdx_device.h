@@ -50,6 +50,7 @@ typedef struct {
     int pad;
     unsigned long long t_start;     /* the step's first kernel */
     unsigned long long t_layers;    /* end of the one launch, or start of the lm_head kernel */
+    unsigned long long t_head;      /* end of the lm_head kernel */
     unsigned long long t_end;       /* when done was set */
 } mdx_host_res;
 
@@ -148,8 +149,8 @@ int mdx_launch_attn_decode(const mdx_state* state, const float* qkv, const float
  * w->kind: MDX_W_I8 (fp16 activations, the NPU path), MDX_W_F16 with fp32
  * activations (the CPU fp16 GEMV), MDX_W_F32 (fp32 rows).  scratch:
  * mdx_lmhead_scratch_bytes() zero bytes (left zero by the kernel).  res (may
- * be NULL): argmax and t_layers, the time the kernel started; logits may be
- * pinned memory. */
+ * be NULL): argmax, t_layers and t_head, the times the kernel started and
+ * ended; logits may be pinned memory. */
 size_t mdx_lmhead_scratch_bytes(void);
 int mdx_launch_lmhead(const float* hidden, const float* norm_w, float eps, const mdx_wdesc* w,
                       float* logits, void* scratch, mdx_state* state, int* out_tokens, int advance,

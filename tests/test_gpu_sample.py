@@ -16,6 +16,8 @@ import os
 import numpy as np
 import pytest
 
+from conftest import tiny_config
+
 pytestmark = pytest.mark.gpu
 
 V_FULL = 151936
@@ -165,3 +167,21 @@ def test_top_k_floor_and_nan_as_the_reference(mdx, gpu, oracle_lib, k):
     z[[10, 20]] = -np.inf
     tok = _check(mdx, oracle_lib, z, top_k=k, u=0.3)
     assert tok == 0
+
+
+def test_sampling_time_is_not_the_lm_heads(mdx, gpu, workdir):
+    """lm_head_ms is the lm_head's own time: a step that samples and returns
+    its logits (a 600 KB copy and two more kernels, 30 us) adds nothing to it."""
+    cfg, d = tiny_config(mdx, vocab_size=151936)
+    path = os.path.join(workdir, "lm_time")
+    mdx.write_model(path, cfg, 1, 5)
+    g = mdx.Decoder(path, cfg, "int8", 64)
+    plain, drawn = [], []
+    for _ in range(12):
+        assert g.step(3)[0] >= 0
+        plain.append(g.stats()["lm_head_ms"])
+        assert g.step_sample(3, 0.5, top_k=50, top_p=0.9, temperature=0.8, logits=True)[0] >= 0
+        drawn.append(g.stats()["lm_head_ms"])
+        assert g.stats()["convert_ms"] > 0
+    # (a plain step's head also stores the logits over the bus)
+    assert 0 < min(drawn) < min(plain) + 0.008
