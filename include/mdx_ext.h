@@ -71,7 +71,7 @@ int mdx_debug_persist_poison_retry(MatmulDecoderContext* ctx);
 /* Test hook (process-wide): on != 0 makes the batch-prefill projections use
  * the GEMM that loads its activation fragments per wave in rounds instead of
  * the one that stages the block's activation panel in LDS (same sums, bit for
- * bit); takes effect for graphs captured afterwards.  Returns the previous
+ * bit); takes effect for prefills that start afterwards.  Returns the previous
  * setting. */
 int mdx_debug_gemm_rounds(int on);
 /* The K-split count of a batch-prefill projection that is split over blocks
@@ -126,8 +126,10 @@ int mdx_generate_greedy(MatmulDecoderContext* ctx, int first_token, int n_steps,
  * repetition. */
 int mdx_time_projection(MatmulDecoderContext* ctx, const char* which, int iters, float* avg_us,
                         double* bytes);
-/* Device milliseconds of one M-row batch prefill through all layers (timed
- * with HIP events, KV position restored afterwards). */
+/* Milliseconds of one M-row batch prefill through all layers, with the rows
+ * and the state on their way up, launched as matmul_decoder_prefill_batch
+ * launches it (timed with HIP events over iters in a row, KV position restored
+ * afterwards). */
 int mdx_time_prefill(MatmulDecoderContext* ctx, const float* embeddings, int M, int iters,
                      float* avg_ms);
 

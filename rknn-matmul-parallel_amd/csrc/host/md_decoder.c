@@ -28,11 +28,6 @@ typedef struct {
     uint16_t *kc, *vc;
 } md_layer;
 
-typedef struct {
-    int M;
-    void* exec;
-} md_pgraph;
-
 #define UP_SLOTS 8
 #define UP_BYTES (1 << 20)
 
@@ -66,9 +61,6 @@ struct MatmulDecoderContext {
     uint16_t *d_bx16, *d_battn16, *d_bact16;
     void *g_layers, *g_step, *g_greedy;
     int graphs_ready;
-    md_pgraph pgraphs[4];
-    int pgraph_next;
-    int capture_M;
     int use_graphs;          /* 0 when MDX_GRAPHS=0: same kernels, launched one by one */
     int persist;             /* 1: the layers of a decode step run as one launch */
     int persist_head;        /* 1: that launch also runs the INT8 lm_head and the argmax */
@@ -669,25 +661,6 @@ static int ensure_graphs(MatmulDecoderContext* c) {
     return 0;
 }
 
-static int seq_prefill(MatmulDecoderContext* c, void* s) { return run_prefill(c, c->capture_M, s); }
-
-static void* prefill_graph(MatmulDecoderContext* c, int M) {
-    if (!c->use_graphs) return NULL;
-    for (int i = 0; i < 4; i++)
-        if (c->pgraphs[i].exec && c->pgraphs[i].M == M) return c->pgraphs[i].exec;
-    md_pgraph* slot = &c->pgraphs[c->pgraph_next];
-    c->pgraph_next = (c->pgraph_next + 1) % 4;
-    if (slot->exec) mdxrt_graph_destroy(slot->exec);
-    slot->exec = NULL;
-    c->capture_M = M;
-    if (capture(c, seq_prefill, &slot->exec) != 0) {
-        slot->exec = NULL;
-        return NULL;
-    }
-    slot->M = M;
-    return slot->exec;
-}
-
 /* ------------------------------------------------------------------------ */
 /* Persistent step                                                           */
 /* ------------------------------------------------------------------------ */
@@ -1087,7 +1060,6 @@ void matmul_decoder_destroy(MatmulDecoderContext* c) {
     mdxrt_graph_destroy(c->g_layers);
     mdxrt_graph_destroy(c->g_step);
     mdxrt_graph_destroy(c->g_greedy);
-    for (int i = 0; i < 4; i++) mdxrt_graph_destroy(c->pgraphs[i].exec);
     mdxrt_free(c->d_tokens);
     mdxrt_free(c->d_trace);
     free(c->h_trace);
@@ -1727,8 +1699,6 @@ int mdx_time_prefill(MatmulDecoderContext* c, const float* embeddings, int M, in
                      float* avg_ms) {
     if (!c || !embeddings || M <= 0 || M > c->max_m || iters <= 0) return MATMUL_DECODER_ERR_INVALID_ARG;
     if (c->seq_len + M > c->max_seq) return MATMUL_DECODER_ERR_INVALID_ARG;
-    void* g = prefill_graph(c, M);
-    if (!g && c->use_graphs) return MATMUL_DECODER_ERR_RKNN;
     memcpy(c->h_io, embeddings, (size_t)M * c->d * 4);
     memset(c->h_state, 0, sizeof(mdx_state));
     c->h_state->pos = c->seq_len;
@@ -1736,7 +1706,7 @@ int mdx_time_prefill(MatmulDecoderContext* c, const float* embeddings, int M, in
     for (int i = 0; i < iters && !rc; i++) {
         rc = mdxrt_h2d_async(c->d_bhidden, c->h_io, (size_t)M * c->d * 4, c->stream);
         if (!rc) rc = mdxrt_h2d_async(c->d_state, c->h_state, sizeof(mdx_state), c->stream);
-        if (!rc) rc = g ? mdxrt_graph_launch(g, c->stream) : run_prefill(c, M, c->stream);
+        if (!rc) rc = run_prefill(c, M, c->stream);
     }
     if (!rc) rc = mdxrt_event_record(c->ev1, c->stream);
     if (!rc) rc = mdxrt_stream_sync(c->stream);

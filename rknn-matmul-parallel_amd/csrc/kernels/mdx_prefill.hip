@@ -932,8 +932,8 @@ size_t mdx_gemm_scratch_floats(int M, int N, int K) {
 
 
 // Test hook: 1 selects k_gemm (fragments loaded in rounds) where k_gemm_p
-// would serve.  Not thread-safe: set it before the contexts it is meant for
-// capture their prefill graphs.
+// would serve.  Not thread-safe: read at every prefill launch, so set it while
+// no other thread prefills.
 static int g_gemm_rounds = 0;
 
 static int gemm_launch(const uint16_t* x16, int M, const mdx_wdesc* w, int epilogue, void* out,

@@ -68,6 +68,9 @@ int mdxrt_event_destroy(void* e) { free(e); return 0; }
 int mdxrt_event_record(void* e, void* s) { *(int*)e = g_tail; return 0; }
 int mdxrt_event_sync(void* e) { run_to(*(int*)e); return 0; }
 int mdxrt_event_elapsed_ms(void* a, void* b, float* ms) { *ms = 1.0f; return 0; }
+int fake_graphs;                          /* captures begun */
+int mdxrt_graph_begin(void* s) { fake_graphs++; return 0; }
+int mdxrt_graph_launch(void* e, void* s) { return 0; }
 int mdxrt_signal(int* flag, unsigned long long* t, void* s) {
     if (fake_fail_signal == 0) return -4;
     if (fake_fail_signal > 0) fake_fail_signal--;

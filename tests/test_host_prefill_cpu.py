@@ -39,6 +39,7 @@ def fake(tmp_path_factory):
     L.matmul_decoder_destroy.argtypes = L.matmul_decoder_clear_kv_cache.argtypes = L.matmul_decoder_get_seq_len.argtypes = [C.c_void_p]
     L.matmul_decoder_prefill_batch.argtypes = [C.c_void_p, F32P, C.c_int]
     L.mdx_prefill_logits.argtypes = [C.c_void_p, F32P, C.c_int, F32P]
+    L.mdx_time_prefill.argtypes = [C.c_void_p, F32P, C.c_int, C.c_int, F32P]
     return L
 
 
@@ -100,5 +101,25 @@ def test_failed_call_leaves_nothing_running(fake, mdx, workdir, n, ok):
         C.c_int.in_dll(fake, "fake_fail_signal").value = -1
         fake.matmul_decoder_clear_kv_cache(h)
         assert fake.mdx_prefill_logits(h, p, n, lp) >= 0 and logits[0] == emb[-1, 0]
+    finally:
+        fake.matmul_decoder_destroy(h)
+
+
+def test_timed_prefill_is_what_callers_run(fake, mdx, workdir):
+    """mdx_time_prefill issues what matmul_decoder_prefill_batch issues, over and
+    over at the same position, and no graph that callers never replay."""
+    h, d = _decoder(fake, mdx, workdir, 256)
+    ms = C.c_float()
+    try:
+        emb, p = _rows(20, d, 5.0)
+        assert fake.matmul_decoder_prefill_batch(h, p, 20) == 0
+        fake.fake_reset()
+        graphs = C.c_int.in_dll(fake, "fake_graphs").value
+        assert fake.mdx_time_prefill(h, p, 20, 3, C.byref(ms)) == 0 and ms.value > 0
+        assert C.c_int.in_dll(fake, "fake_graphs").value == graphs
+        got = np.ctypeslib.as_array((C.c_float * 60).in_dll(fake, "fake_rows"))
+        assert C.c_int.in_dll(fake, "fake_n_rows").value == 60 and np.array_equal(got, np.tile(emb[:, 0], 3))
+        assert list((C.c_int * 3).in_dll(fake, "fake_pos")) == [20, 20, 20]
+        assert fake.matmul_decoder_get_seq_len(h) == 20 and fake.fake_pending() == 0
     finally:
         fake.matmul_decoder_destroy(h)
