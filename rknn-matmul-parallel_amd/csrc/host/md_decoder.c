@@ -879,7 +879,8 @@ static MatmulDecoderContext* create_common(const MatmulDecoderConfig* config,
     int mm = config->max_batch_prefill > 0 ? config->max_batch_prefill : 64;
     c->max_m = mm > 64 ? 64 : mm;
     /* a chunk size below 64 is kept to; otherwise a longer prompt goes in
-     * passes of up to 2048 rows (about 80 MB of activations at d = 1024) */
+     * passes of up to 2048 rows (67 MB of activations and partials at d = 1024,
+     * and 8 MB pinned) */
     c->long_m = c->max_m == 64 && max_seq_len > 64 ? (max_seq_len < 2048 ? max_seq_len : 2048) : 0;
     c->max_splits = mdx_attn_max_splits(max_seq_len);
     {

@@ -307,7 +307,7 @@ int mdx_long_ok(const mdx_wdesc* w);
  * act[M][N/2] of rows [0,N/2) gate and [N/2,N) up. */
 int mdx_launch_long_gemm(const uint16_t* x16, int M, const mdx_wdesc* w, int swiglu, void* out, void* stream);
 /* Residual projection + next RMSNorm, as mdx_launch_gemm_residual_norm;
- * scratch: mdx_long_scratch_floats(M, N) floats. */
+ * scratch: mdx_long_scratch_floats(M, N) floats, enough for fewer rows too. */
 size_t mdx_long_scratch_floats(int M, int N);
 int mdx_launch_long_residual_norm(const uint16_t* x16, int M, const mdx_wdesc* w, float* hidden,
                                   const float* norm_w, float eps, uint16_t* x16_out, float* scratch,

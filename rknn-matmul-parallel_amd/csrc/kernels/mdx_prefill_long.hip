@@ -725,6 +725,11 @@ int cdiv(int a, int b) { return (a + b - 1) / b; }
 // Tiles of 128 x 128 once they fill the chip twice over, else 64-row or 64 x 64
 // ones; the residual projections (which can sum partials) also split K into
 // runs of at least 256 until there are about 512 blocks.
+constexpr int kMaxLongSplits = 8;
+int long_splits(int tiles) {
+    const int ns = 512 / tiles;
+    return ns > kMaxLongSplits ? kMaxLongSplits : (ns < 1 ? 1 : ns);
+}
 LongTile long_tile(int M, int N, int K, bool can_split, bool wide) {
     LongTile t;
     t.splits = 1;
@@ -732,10 +737,9 @@ LongTile long_tile(int M, int N, int K, bool can_split, bool wide) {
     else if (wide) t.bm = 64, t.bn = 128;
     else t.bm = t.bn = 64;
     if (can_split) {
-        const int tiles = cdiv(M, t.bm) * cdiv(N, t.bn), nst = cdiv(K, kKT);
-        int ns = 512 / tiles;
+        const int nst = cdiv(K, kKT);
+        int ns = long_splits(cdiv(M, t.bm) * cdiv(N, t.bn));
         if (ns > K / 256) ns = K / 256;
-        if (ns > 8) ns = 8;
         if (ns < 1) ns = 1;
         const int per = cdiv(nst, ns);
         t.splits = cdiv(nst, per);          // none is empty
@@ -821,10 +825,15 @@ int mdx_launch_long_gemm(const uint16_t* x16, int M, const mdx_wdesc* w, int swi
 }
 
 size_t mdx_long_scratch_floats(int M, int N) {
-    /* splits <= min(8, 512 / tiles), each tile at most 128 x 128 */
-    const size_t mn = (size_t)M * N, cap = (size_t)512 * 128 * 128;
-    const size_t most = 8 * mn < cap ? 8 * mn : cap;
-    return mn > most ? mn : most;
+    /* the most that any launch of up to M rows leaves, whatever its K (hidden
+     * 1024, 2048 rows: 8.4 MB) */
+    size_t most = 0;
+    for (int m = 1; m <= M; m++) {
+        const LongTile t = long_tile(m, N, 256, false, false);
+        const size_t n = (size_t)long_splits(cdiv(m, t.bm) * cdiv(N, t.bn)) * m * N;
+        if (n > most) most = n;
+    }
+    return most;
 }
 
 int mdx_launch_long_residual_norm(const uint16_t* x16, int M, const mdx_wdesc* w, float* hidden,

@@ -105,6 +105,21 @@ def test_failed_call_leaves_nothing_running(fake, mdx, workdir, n, ok):
         fake.matmul_decoder_destroy(h)
 
 
+def test_split_partials_of_long_prompts(mdx):
+    """The partials' scratch holds every launch of up to M rows and little more
+    (hidden 1024, passes of 2048 rows: 8.4 MB)."""
+    need = mdx.lib().mdx_long_scratch_floats
+    need.restype = C.c_size_t
+    assert need(2048, 1024) * 4 <= 8.5e6
+    for N in (32, 160, 1024, 1536, 2048, 5120, 16384):
+        for M in (65, 127, 128, 203, 515, 1000, 1024, 2000, 2048):
+            for m in (1, 64, M // 2, M - 1, M):
+                # 128 x 128 tiles from 256 of them on, else 64 x 64; up to 8 splits while there are fewer than 512 blocks
+                t = 128 if -(-m // 128) * -(-N // 128) >= 256 else 64
+                splits = max(1, min(8, 512 // (-(-m // t) * -(-N // t))))
+                assert need(M, N) >= splits * m * N, (M, N, m)
+
+
 def test_timed_prefill_is_what_callers_run(fake, mdx, workdir):
     """mdx_time_prefill issues what matmul_decoder_prefill_batch issues, over and
     over at the same position, and no graph that callers never replay."""
