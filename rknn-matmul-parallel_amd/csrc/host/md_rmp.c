@@ -190,6 +190,18 @@ static int rmp_collect(RmpContext* c, float* output, int p) {
 int rmp_run(RmpContext* c, const int16_t* input, float* output) {
     if (!c || !input || !output) return -1;
     const int passes = (c->config.M + c->rows - 1) / c->rows;
+    int16_t* own = NULL;
+    if (passes > c->slots) {
+        /* the first passes' rows are stored before the last ones are read: a
+         * caller's output may lie over its input */
+        const size_t nx = (size_t)c->config.M * c->config.K * 2, ny = (size_t)c->config.M * c->config.N * 4;
+        if ((uintptr_t)input < (uintptr_t)output + ny && (uintptr_t)output < (uintptr_t)input + nx) {
+            own = (int16_t*)malloc(nx);
+            if (!own) return -1;
+            memcpy(own, input, nx);
+            input = own;
+        }
+    }
     int rc = 0, done = 0;
     for (int p = 0; p < passes && !rc; p++) {
         if (p >= c->slots) rc = rmp_collect(c, output, done++);
@@ -200,6 +212,7 @@ int rmp_run(RmpContext* c, const int16_t* input, float* output) {
         mdxrt_stream_sync(c->stream[0]);
         if (c->stream[1]) mdxrt_stream_sync(c->stream[1]);
     }
+    free(own);
     return rc ? -1 : 0;
 }
 

@@ -32,3 +32,24 @@ def test_rmp_passes(mdx, gpu, M, K, N):
             assert rel_err(y, x.astype(np.float64) @ w.astype(np.float64)) < 1e-5
     finally:
         L.rmp_destroy(h)
+
+
+def test_rmp_output_over_input(mdx, gpu):
+    """Input rows at the start of the output buffer, eight passes through four
+    slots: the first passes' rows are stored before the last are read."""
+    M, K, N = 900, 64, 4098
+    rng = np.random.default_rng(1)
+    w = (rng.standard_normal((K, N)) * 0.02).astype(np.float16)
+    x = rng.standard_normal((M, K)).astype(np.float16)
+    y = np.zeros((M, N), np.float32)
+    L = mdx.lib()
+    h = L.rmp_create(C.byref(mdx.RmpConfig(M, K, N, 0, 0, 2)), w.ctypes.data, None)
+    assert h
+    try:
+        for at in (0, M * N * 4 - x.nbytes, 4 * N * 500):
+            y.view(np.uint8).ravel()[at:at + x.nbytes] = x.view(np.uint8).ravel()
+            xin = C.cast(C.c_void_p(y.ctypes.data + at), mdx._U16)
+            assert L.rmp_run(h, xin, y.ctypes.data_as(mdx._F)) == 0
+            assert rel_err(y, x.astype(np.float64) @ w.astype(np.float64)) < 1e-5
+    finally:
+        L.rmp_destroy(h)
