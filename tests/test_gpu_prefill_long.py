@@ -199,3 +199,46 @@ def test_long_prefill_decoder(mdx, gpu, oracle_lib, workdir, quant, over):
     to, lo = o.step(5)
     assert tg == to and rel_err(lg, lo) < 1e-3 and cosine(lg, lo) > 0.9999
     assert g.seq_len == o.seq_len == 202
+
+
+def _prompts_and_a_step(mdx, oracle_lib, path, cfg, d, max_seq, prompts, rows):
+    """Prompts one behind the other, then a step: last-row logits and the given
+    cache rows against the oracle."""
+    g = mdx.Decoder(path, cfg, "fp16", max_seq)
+    o = oracle_lib.Model(path, d, 0, max_seq, kv_fp16=True)
+    rng = np.random.default_rng(4)
+    for n in prompts:
+        emb = rng.standard_normal((n, d["hidden_dim"])).astype(np.float32)
+        tok, lg = g.prefill_logits(emb)
+        assert o.prefill_batch(emb) == 0 and tok >= 0
+        x16 = oracle_lib.f16_to_f32(oracle_lib.f32_to_f16(o.last_normed())).astype(np.float64)
+        hq, hs = o.lm_head_q()
+        assert rel_err(lg, (hq.astype(np.float64) @ x16) * hs) < 1e-3
+    for layer in range(d["num_layers"]):
+        for at, n in rows:
+            for a, b in zip(g.kv_read(layer, at, n), o.kv_read(layer, at, n)):
+                assert rel_err(a, b) < 2e-3
+    tg, lg = g.step(5)
+    to, lo = o.step(5)
+    assert tg == to and rel_err(lg, lo) < 1e-3 and g.seq_len == o.seq_len == sum(prompts) + 1
+
+
+@pytest.mark.parametrize("over", [dict(), dict(num_q_heads=4, num_kv_heads=1, head_dim=256)])
+def test_long_prefill_in_passes(mdx, gpu, oracle_lib, workdir, over):
+    """2300 rows (two passes of 1150, which reuse the activations and the
+    upload ring; head_dim 256 takes its position from the device), and 2100
+    more behind them: the rows on both sides of every pass's end."""
+    cfg, d = tiny_config(mdx, max_seq_len=4500, num_layers=1, **over)
+    path = os.path.join(workdir, "passes_%d" % d["head_dim"])
+    mdx.write_model(path, cfg, 0, 78)
+    _prompts_and_a_step(mdx, oracle_lib, path, cfg, d, 4500, (2300, 2100), [(0, 4), (1100, 100), (2290, 20), (3340, 20), (4390, 10)])
+
+
+@pytest.mark.parametrize("chunk,prompts", [(16, (70, 16, 1)), (63, (127, 64)), (1, (5,))])
+def test_prefill_in_short_chunks(mdx, gpu, oracle_lib, workdir, chunk, prompts):
+    """A max_batch_prefill below 64 is kept to, whatever the prompt's length."""
+    cfg, d = tiny_config(mdx, max_seq_len=256, max_batch_prefill=chunk)
+    path = os.path.join(workdir, "chunks")
+    if not os.path.isdir(path):
+        mdx.write_model(path, cfg, 0, 79)
+    _prompts_and_a_step(mdx, oracle_lib, path, cfg, d, 256, prompts, [(0, sum(prompts))])
