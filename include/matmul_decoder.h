@@ -83,7 +83,8 @@ typedef struct {
 
     int disable_npu_lm_head;    /* 1 = fp16-weight lm_head with fp32 activations instead of INT8 */
 
-    int max_batch_prefill;      /* prefill rows per pass: below 64 kept to; 0 or more = the library's choice */
+    int max_batch_prefill;      /* prefill rows per pass: 1..63 are kept to; 0, 64 and more: the
+                                   library's choice (up to 64 rows, then passes of up to 2048) */
 } MatmulDecoderConfig;
 
 /* Qwen3-0.6B defaults (reference: include/matmul_decoder.h:119-144). */

@@ -793,8 +793,8 @@ static int launch_persist(MatmulDecoderContext* c, int head, int* out_tokens, in
 static pthread_mutex_t g_persist_mu = PTHREAD_MUTEX_INITIALIZER;
 
 /* After a timed-out ordinary launch: switch the context to cooperative
- * launches.  Returns 1 when the caller should run the step again (the state
- * is uploaded again; the K/V rows the failed step wrote are rewritten). */
+ * launches.  Returns 1 when the caller should run the step again (it feeds the
+ * same state again; the K/V rows the failed step wrote are rewritten). */
 static int persist_retry(MatmulDecoderContext* c) {
     if (!c->persist || c->persist_coop) return 0;
     c->persist_coop = 1;
@@ -806,8 +806,9 @@ static int persist_retry(MatmulDecoderContext* c) {
      * another grid) read the step counter after workgroup 0 had advanced it,
      * and published words tagged with the epochs the retry would use.  Zeroing
      * the exchange words, the counter with them, leaves no word the retry can
-     * accept before its own writer stores it (epoch 0 is never valid).  The
-     * stream is synchronised, so no workgroup of that launch is still running. */
+     * accept before its own writer stores it (epoch 0 is never valid).  No
+     * workgroup of that launch is still running: the caller has synchronised
+     * the stream or seen the word that is set behind the launch. */
     if (mdxrt_fill_u32(c->d_xbuf, 0u, mdx_persist_xbuf_bytes() / 4, c->stream) ||
         (c->lx_buf && mdxrt_fill_u32(c->lx_buf, 0u, mdx_persist_xbuf_bytes() / 4, c->stream)) ||
         mdxrt_stream_sync(c->stream))

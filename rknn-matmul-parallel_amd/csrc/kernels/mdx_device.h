@@ -46,7 +46,7 @@ typedef struct {
 typedef struct {
     int argmax;
     int timeout;                    /* 1 when a wait of the one-launch step timed out */
-    int done;                       /* set last, by mdxrt_signal or the lm_head */
+    int done;                       /* set last, by mdxrt_signal */
     int pad;
     unsigned long long t_start;     /* the step's first kernel */
     unsigned long long t_layers;    /* end of the one launch, or start of the lm_head kernel */

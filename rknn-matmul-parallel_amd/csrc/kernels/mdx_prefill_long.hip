@@ -5,10 +5,10 @@
 // enough rows to tile both operands: here the projections are LDS-tiled MFMA
 // GEMMs over all rows (each weight read once per row tile, int8/int4 widened
 // to fp16 once per block as they are staged), and attention runs 64 query
-// rows of one KV head against each staged K/V tile on MFMA.  A prompt of 2000
-// rows through 28 fp16 layers (hidden 1024) and 32 tokens: 91.0 -> 23.3 ms;
-// 4000 rows through 2 int4 layers and 32 tokens: 20.1 -> 4.1 ms; 203 rows
-// through 4 int8 layers and 16 tokens: 2.23 -> 1.77 ms.
+// rows of one KV head against each staged K/V tile on MFMA.  A prompt alone,
+// through 4 layers of hidden 1024, against chunks of 64 rows: fp16 65 rows 381
+// -> 240 us, 200 853 -> 317, 1500 7783 -> 960; int4 65 337 -> 262, 1500 7381
+// -> 1020.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -382,12 +382,12 @@ __global__ __launch_bounds__(256, 2) void k_long_gemm(LongArgs a) {
 // take alternate K/V tiles of 64 positions and are merged at the end: the
 // causal rows make the last blocks twice as long as the average one, and
 // nothing else is left to run beside them, so a block's own length is what
-// counts (one group, two blocks per CU: 67 us at M = 2000, 55 with two).
-// Tiles are staged in LDS (V transposed), the group's next one in registers
-// meanwhile.  S^T = K . Q^T,
-// so a lane holds scores of one query row and its running maximum and sum are
-// its own; P^T is then already the B operand of O^T = V^T . P^T (the k order
-// of that product is the order in which a lane holds its scores).
+// counts (one group, two blocks per CU: 67 us at M = 2000 within a prefill, 55
+// with two).  Tiles are staged in LDS (V transposed), the group's next one in
+// registers meanwhile.  S^T = K . Q^T, so a lane holds scores of one query row
+// and its running maximum and sum are its own; P^T is then already the B operand
+// of O^T = V^T . P^T (the k order of that product is the order in which a lane
+// holds its scores).
 //
 // Queries and probabilities are fp32: each goes in as the sum of two fp16
 // values, both rounded to nearest (23 bits), the queries scaled per row so that
@@ -400,8 +400,9 @@ __global__ __launch_bounds__(256, 2) void k_long_gemm(LongArgs a) {
 // otherwise than the exact result rounds, per thousand, before these / now /
 // k_attn_prefill, normal inputs, 16 heads of 128 over 8: M = 515 1.87 / 0.98 /
 // 1.03, M = 2000 2.11 / 1.11 / 1.16, equal scores 1.13 / 0.49 / 0.62; 8 of 256
-// over 2, M = 515: 2.10 / 0.98 / 0.98.  Their cost at M = 2000: 69.3 -> 70.2
-// us; 256 dimensions 159 -> 135 us (independent sums).
+// over 2, M = 515: 2.10 / 0.98 / 0.98.  Their cost, launched alone on cold
+// inputs, M = 2000: 69.3 -> 70.2 us; 256 dimensions 159 -> 135 us (independent
+// sums).
 //
 // The vector unit is what bounds it (at M = 2000 the longest block's tile took
 // 2.9 us with expf and a rescale per tile): the exponentials are v_exp_f32 of
@@ -722,9 +723,16 @@ struct LongTile {
 
 int cdiv(int a, int b) { return (a + b - 1) / b; }
 
-// Tiles of 128 x 128 once they fill the chip twice over, else 64-row or 64 x 64
-// ones; the residual projections (which can sum partials) also split K into
-// runs of at least 256 until there are about 512 blocks.
+// Tiles of 128 x 128 once there are 256 of them, one per CU, else 64-row or 64
+// x 64 ones; the residual projections (which can sum partials) also split K
+// into runs of at least 256 until there are about 512 blocks.  64 x 64 / 128 x
+// 128, us: fp16 K = 1024, N = 4096: M = 512 (128 tiles of 128) 14.8 / 22.4, 896
+// (224) 23.5 / 24.2, 1024 (256) 24.3 / 24.7, 1500 (384) 32.9 / 30.2, 2000 (512)
+// 42.1 / 31.5; N = 6144: 640 (240) 24.2 / 24.4, 896 (336) 32.2 / 30.5, 2000
+// (768) 62.2 / 53.7.  int8 and int4 break even later: int8 N = 4096 1024 (256)
+// 24.2 / 27.8, 1500 33.2 / 33.0, 2000 42.1 / 33.7.  The tile is chosen before
+// the split: N = 1024 with split and norm, fp16 K = 3072: M = 1000 (64) 24.9 /
+// 27.6, 2000 (128) 40.8 / 36.6; K = 2048 20.3 / 25.8, 31.1 / 31.1.
 constexpr int kMaxLongSplits = 8;
 int long_splits(int tiles) {
     const int ns = 512 / tiles;
